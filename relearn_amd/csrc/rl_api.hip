@@ -334,7 +334,7 @@ int init_networks(rl_bh_ctx* c, uint32_t G, const uint64_t* offsets, const doubl
     RL_TRY(dalloc(c, &c->searched, n));
     RL_TRY(dalloc(c, &c->coop_flag, n));
     RL_TRY(dalloc(c, &c->coop_work, n));
-    RL_TRY(dalloc(c, &c->coop_cursor, kCursorSlots));
+    RL_TRY(dalloc(c, &c->coop_cursor, kCursorSlots * kCursorStride));
     RL_TRY(dalloc(c, &c->coop_overflow, n));
     RL_TRY(dalloc(c, &c->redo, n));
     {

@@ -489,7 +489,7 @@ __global__ void k_search_reset(uint64_t n, const uint64_t* __restrict__ slot_tot
         }
     }
     if (t0 < kCursorSlots) {
-        cursor[t0] = 0;
+        cursor[t0 * kCursorStride] = 0;
     }
 }
 

@@ -631,28 +631,27 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8
     const uint32_t q = ln >> 3U, j = ln & 7U;
     const uint64_t base = static_cast<uint64_t>(blockIdx.x) * a.cap;
     int seg = static_cast<int>(blockIdx.x % kXcds);
-    int tried = 0;
     unsigned long long acc_exec = 0;
     const uint64_t nw = *a.nwork;
     if (nw >= a.run_below) {
         return;   // the group walk takes this update
     }
     const uint32_t step = *s.step;
-    const uint32_t chunk = a.chunk;
+    const uint32_t chunk = grab_size(nw, a.chunk);
     uint64_t w_next = 0, w_lim = 0;   // the wave's current chunk of its segment
     while (true) {
         if (w_next >= w_lim) {
             const uint64_t seg_end = nw * static_cast<uint64_t>(seg + 1) / kXcds;
             uint64_t w0 = 0;
             if (ln == 0) {
-                w0 = nw * static_cast<uint64_t>(seg) / kXcds + atomicAdd(&a.cursor[seg], static_cast<unsigned long long>(chunk));
+                w0 = nw * static_cast<uint64_t>(seg) / kXcds + atomicAdd(&a.cursor[seg * kCursorStride], static_cast<unsigned long long>(chunk));
             }
             w0 = __shfl(w0, 0, kWave);
             if (w0 >= seg_end) {
-                if (++tried >= kXcds) {
+                seg = next_segment(a.cursor, nw, seg);
+                if (seg < 0) {
                     break;
                 }
-                seg = (seg + 1) % kXcds;
                 continue;
             }
             w_next = w0;
@@ -728,7 +727,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8
         }
         __syncthreads();
     }
-    if (ln == 0) {
+    if (ln == 0 && acc_exec != 0) {
         atomicAdd(&s.counters[kCtrTestsExec], acc_exec);
     }
 }

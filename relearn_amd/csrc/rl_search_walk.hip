@@ -355,7 +355,6 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(6, 6
     double* const tcum = a.t_cum + cbase * kWave;
     uint32_t* const tchild = a.t_child + cbase * 8;
     int seg_x = static_cast<int>(blockIdx.x % kXcds);
-    int tried = 0;
     unsigned long long acc_exec = 0;
     const uint64_t nw = a.seg_goff[a.nseg];
     const uint32_t step = *s.step;
@@ -372,15 +371,15 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(6, 6
             uint64_t w0 = 0;
             if (ln == 0) {
                 w0 = nw * static_cast<uint64_t>(seg_x) / kXcds +
-                     atomicAdd(&a.cursor[seg_x], static_cast<unsigned long long>(chunk));
+                     atomicAdd(&a.cursor[seg_x * kCursorStride], static_cast<unsigned long long>(chunk));
             }
             w0 = (static_cast<uint64_t>(uniform_u32(static_cast<uint32_t>(w0 >> 32U))) << 32U) |
                  uniform_u32(static_cast<uint32_t>(w0));
             if (w0 >= seg_end) {
-                if (++tried >= kXcds) {
+                seg_x = next_segment(a.cursor, nw, seg_x);
+                if (seg_x < 0) {
                     break;
                 }
-                seg_x = (seg_x + 1) % kXcds;
                 continue;
             }
             w_next = w0;
