@@ -33,7 +33,7 @@ enum {
 };
 
 enum {
-    RL_PREC_FP64 = 0,        /* all arithmetic in IEEE binary64, same operation order as the CPU path */
+    RL_PREC_FP64 = 0,        /* all arithmetic in IEEE binary64; decisions as the CPU path makes them */
     RL_PREC_FP32_MIXED = 1,  /* FP32 distances and Gaussian; FP64 centroids, sums and prefix sums */
 };
 

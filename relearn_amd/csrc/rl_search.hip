@@ -621,6 +621,7 @@ SearchArgs search_args(rl_bh_ctx* c) {
         a.meta[k] = c->tree.meta[k];
     }
     a.theta = c->cfg.theta;
+    a.theta2 = c->cfg.theta * c->cfg.theta;
     a.scale64 = -1.0 / (c->cfg.sigma * c->cfg.sigma);
     a.mu = c->cfg.mu;
     a.theta2f = static_cast<float>(c->cfg.theta * c->cfg.theta);

@@ -69,6 +69,7 @@ struct CoopShared {
     uint32_t stage_fx[kStageCap + 1];  // first expanded child slot | count << 28 of slot i at i % kStageCap
     double stage_ms[kStageCap + 1];    // probability mass of slot i at i % kStageCap
     uint32_t lvl_start[kMaxLevels + 4];
+    double2 exp_table[32];             // 2^(i/32), first and second part (FP64 search only)
 };
 
 __device__ __forceinline__ uint32_t lane() {
@@ -156,30 +157,107 @@ __device__ __forceinline__ NodeData load_node(const Lane& L, uint32_t node, bool
     return d;
 }
 
+// 2^(i/32), i = 0..31, each as the nearest FP64 number and the nearest one to the rest.
+__constant__ const double kExpTable[32][2] = {
+    { 0x1.0000000000000p+0, 0x0.0p+0 },
+    { 0x1.059b0d3158574p+0, 0x1.d73e2a475b465p-55 },
+    { 0x1.0b5586cf9890fp+0, 0x1.8a62e4adc610bp-54 },
+    { 0x1.11301d0125b51p+0, -0x1.6c51039449b3ap-54 },
+    { 0x1.172b83c7d517bp+0, -0x1.19041b9d78a76p-55 },
+    { 0x1.1d4873168b9aap+0, 0x1.e016e00a2643cp-54 },
+    { 0x1.2387a6e756238p+0, 0x1.9b07eb6c70573p-54 },
+    { 0x1.29e9df51fdee1p+0, 0x1.612e8afad1255p-55 },
+    { 0x1.306fe0a31b715p+0, 0x1.6f46ad23182e4p-55 },
+    { 0x1.371a7373aa9cbp+0, -0x1.63aeabf42eae2p-54 },
+    { 0x1.3dea64c123422p+0, 0x1.ada0911f09ebcp-55 },
+    { 0x1.44e086061892dp+0, 0x1.89b7a04ef80d0p-59 },
+    { 0x1.4bfdad5362a27p+0, 0x1.d4397afec42e2p-56 },
+    { 0x1.5342b569d4f82p+0, -0x1.07abe1db13cadp-55 },
+    { 0x1.5ab07dd485429p+0, 0x1.6324c054647adp-54 },
+    { 0x1.6247eb03a5585p+0, -0x1.383c17e40b497p-54 },
+    { 0x1.6a09e667f3bcdp+0, -0x1.bdd3413b26456p-54 },
+    { 0x1.71f75e8ec5f74p+0, -0x1.16e4786887a99p-55 },
+    { 0x1.7a11473eb0187p+0, -0x1.41577ee04992fp-55 },
+    { 0x1.82589994cce13p+0, -0x1.d4c1dd41532d8p-54 },
+    { 0x1.8ace5422aa0dbp+0, 0x1.6e9f156864b27p-54 },
+    { 0x1.93737b0cdc5e5p+0, -0x1.75fc781b57ebcp-57 },
+    { 0x1.9c49182a3f090p+0, 0x1.c7c46b071f2bep-56 },
+    { 0x1.a5503b23e255dp+0, -0x1.d2f6edb8d41e1p-54 },
+    { 0x1.ae89f995ad3adp+0, 0x1.7a1cd345dcc81p-54 },
+    { 0x1.b7f76f2fb5e47p+0, -0x1.5584f7e54ac3bp-56 },
+    { 0x1.c199bdd85529cp+0, 0x1.11065895048ddp-55 },
+    { 0x1.cb720dcef9069p+0, 0x1.503cbd1e949dbp-56 },
+    { 0x1.d5818dcfba487p+0, 0x1.2ed02d75b3707p-55 },
+    { 0x1.dfc97337b9b5fp+0, -0x1.1a5cd4f184b5cp-54 },
+    { 0x1.ea4afa2a490dap+0, -0x1.e9c23179c2893p-54 },
+    { 0x1.f50765b6e4540p+0, 0x1.9d3e12dd8a18bp-54 },
+};
+
+// Lanes that accept, and lanes that expand, their node.
+struct Verdict {
+    uint64_t accept, expand;
+};
+
+// Below this a squared distance, or a list's probability sum, is left to the formulas of the CPU path:
+// squares of distances under about 1e-125 lose bits to underflow, and so do probabilities near the
+// smallest FP64 numbers, whose sums then depend on how the exponent was rounded.
+constexpr double kTiny = 1.0e-250;
+
+// exp(x) of a Gaussian exponent (x <= 0) in FP64.
+//   x = (32 e + i) ln2/32 + r,  exp(x) = 2^e 2^(i/32) exp(r),  |r| <= ln2/64
+// with ln2/32 in two parts (the fused x - k ln2/32 of the first is exact), 2^(i/32) in two parts from the
+// table, and the Taylor polynomial of exp(r) - 1 to r^6 (the next term is below 4e-18).  Largest error
+// against 64-bit-mantissa values at 2 million points of [-700, 0]: 0.55 units in the last place (the math
+// library's exp: 0.86); about 20 vector instructions instead of 34.
+__device__ __forceinline__ double exp_gauss(double x, const double2* table) {
+#pragma clang fp contract(off)
+    const double k = __builtin_rint(x * 46.16624130844683);
+    double r = __builtin_fma(k, -0x1.62e42fefa39efp-6, x);
+    r = __builtin_fma(k, -0x1.abc9e3b39803fp-61, r);
+    const int n = static_cast<int>(k);
+    const double2 t = table[n & 31];
+    double q = __builtin_fma(r, 1.0 / 720.0, 1.0 / 120.0);
+    q = __builtin_fma(r, q, 1.0 / 24.0);
+    q = __builtin_fma(r, q, 1.0 / 6.0);
+    q = __builtin_fma(r, q, 0.5);
+    q = __builtin_fma(r * r, q, r);
+    return ldexp(t.x + __builtin_fma(t.x, q, t.y), n >> 5);
+}
+
 // Acceptance test and probability of a loaded node (test_acceptance_criterion, BarnesHutBase.h:72-114;
-// Kernel::calculate_attractiveness_to_connect, Kernel.h:61-75) for the lanes with `act`; other lanes
-// return kDiscard and p = 0.  The FP32 path is branch-free; exact coincidences and decisions inside
-// the guard band are redone in FP64 under one wave-uniform branch.
+// Kernel::calculate_attractiveness_to_connect, Kernel.h:61-75) for the lanes in `act`; p = 0 in lanes
+// that do not accept.  The verdicts are lane masks combined in scalar registers, which the scalar unit
+// does beside the vector arithmetic that bounds the kernel.
+//
+// Both precisions decide on squares, side^2 against theta^2 d^2, and leave what is too close (and
+// distances of 0) to the reference's own comparison under one wave-uniform branch.  FP32: exact
+// fixed-point differences, a leaf's squared side is -infinity, hence accepted.  FP64: a relative margin
+// of 1e-13, a thousand times the rounding of both sides, so a decision outside it is the
+// reference's; the Gaussian takes d^2 itself, which is rounded less than the square of the reference's
+// scaled hypot.  That hypot (three divisions and a square root, about 75 of the 210 vector
+// instructions of an FP64 step) and the library's exp made the FP64 search of 1M neurons 24.4 ms; with
+// squares and exp_gauss it takes 16.0 ms.
 template <bool kMixed, bool kMu0>
-__device__ __forceinline__ int eval_node(const SearchArgs& a, const Lane& L, const NodeData& d, uint32_t node, bool act,
-                                         double* p_out) {
+__device__ __forceinline__ Verdict eval_node(const SearchArgs& a, const Lane& L, const NodeData& d, uint32_t node,
+                                             uint64_t act, const double2* table, double* p_out) {
+#pragma clang fp contract(off)
     // The source's own leaf lies at distance 0 and is discarded by the test, so the kernel's
     // self-exclusion (Kernel.h:61-75) never applies here.
-    const bool valid = act && d.m.x != 0;
-    const bool leaf = (d.m.y >> kLinkBits) == 0;
+    const uint64_t valid = act & __builtin_amdgcn_ballot_w64(d.m.x != 0);
+    Verdict v;
+    uint64_t unsure;
+    double p;
     if (kMixed) {
-        const int32_t ix = static_cast<int32_t>(d.r32.x) - L.qx;
-        const int32_t iy = static_cast<int32_t>(d.r32.y) - L.qy;
-        const int32_t iz = static_cast<int32_t>(d.r32.z) - L.qz;
-        const float dx = static_cast<float>(ix);
-        const float dy = static_cast<float>(iy);
-        const float dz = static_cast<float>(iz);
+        const float dx = static_cast<float>(static_cast<int32_t>(d.r32.x) - L.qx);
+        const float dy = static_cast<float>(static_cast<int32_t>(d.r32.y) - L.qy);
+        const float dz = static_cast<float>(static_cast<int32_t>(d.r32.z) - L.qz);
         const float d2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
         const float s2 = __uint_as_float(d.r32.w);
         const float g = __builtin_fmaf(a.theta2f, d2, -s2);
-        const bool coinc = (ix | iy | iz) == 0;
-        const bool near = !leaf && fabsf(g) <= __builtin_fmaf(a.guard, s2, a.guard_abs);
-        int st = (leaf || g > 0.0f) ? kAccept : kExpand;
+        // the squared distance of integer differences is 0 exactly at a coincidence
+        const uint64_t coinc = __builtin_amdgcn_ballot_w64(d2 == 0.0f);
+        const uint64_t near = __builtin_amdgcn_ballot_w64(fabsf(g) <= __builtin_fmaf(a.guard, s2, a.guard_abs));
+        const uint64_t pos = __builtin_amdgcn_ballot_w64(g > 0.0f);
         float x;
         if (kMu0) {
             x = d2 * L.k2q;
@@ -188,32 +266,51 @@ __device__ __forceinline__ int eval_node(const SearchArgs& a, const Lane& L, con
             x = dd * dd * a.k2f;
         }
         const float w = __builtin_amdgcn_exp2f(x) * static_cast<float>(d.m.x);
-        double p = static_cast<double>(w);
-        st = valid ? st : kDiscard;
-        p = st == kAccept ? p : 0.0;
-        const bool need = valid && (coinc || near);
-        if (__builtin_amdgcn_ballot_w64(need) != 0) {
-            if (need) {
-                const Eval e = eval_exact(a, L, node, 0, leaf);
-                st = e.status;
-                p = st == kAccept ? probability<false>(a, L, e, d.m.x, kGauss) : 0.0;
-            }
-        }
-        *p_out = p;
-        return st;
+        unsure = valid & (coinc | near);
+        v.accept = valid & ~unsure & pos;
+        v.expand = valid & ~unsure & ~pos;
+        float wa = __builtin_amdgcn_inverse_ballot_w64(v.accept) ? w : 0.0f;
+        __asm__ volatile("" : "+v"(wa));   // select in FP32, then one conversion
+        p = static_cast<double>(wa);
     } else {
-        double p = 0.0;
+        const double dx = d.r64.x - L.px;
+        const double dy = d.r64.y - L.py;
+        const double dz = d.r64.z - L.pz;
+        const double d2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
+        const double t = a.theta2 * d2;
+        const double s2 = d.r64.w * d.r64.w;
+        const uint64_t leaf = __builtin_amdgcn_ballot_w64((d.m.y >> kLinkBits) == 0);
+        const uint64_t above = leaf | __builtin_amdgcn_ballot_w64(s2 < t * (1.0 - 1.0e-13));
+        const uint64_t below = __builtin_amdgcn_ballot_w64(s2 > t * (1.0 + 1.0e-13));
+        unsure = valid & (__builtin_amdgcn_ballot_w64(!(d2 > kTiny)) | ~(above | below));
+        v.accept = valid & ~unsure & above;
+        v.expand = valid & ~unsure & ~above;
+        double x;
+        if (kMu0) {
+            x = d2 * a.scale64;
+        } else {
+            const double dd = sqrt(d2) - a.mu;
+            x = (dd * dd) * a.scale64;
+        }
+        // exp is 0 below -745.2; the clamp keeps the exponent arithmetic in range
+        const double w = exp_gauss(fmax(x, -800.0), table) * static_cast<double>(d.m.x);
+        p = __builtin_amdgcn_inverse_ballot_w64(v.accept) ? w : 0.0;
+    }
+    if (unsure != 0) {
         int st = kDiscard;
-        if (valid) {
-            const Eval e = eval_exact_rec(a, L, d.r64, leaf);
+        if (__builtin_amdgcn_inverse_ballot_w64(unsure)) {
+            const bool leaf = (d.m.y >> kLinkBits) == 0;
+            const Eval e = kMixed ? eval_exact(a, L, node, 0, leaf) : eval_exact_rec(a, L, d.r64, leaf);
             st = e.status;
             if (st == kAccept) {
                 p = probability<false>(a, L, e, d.m.x, kGauss);
             }
         }
-        *p_out = p;
-        return st;
+        v.accept |= __builtin_amdgcn_ballot_w64(st == kAccept);
+        v.expand |= __builtin_amdgcn_ballot_w64(st == kExpand);
     }
+    *p_out = p;
+    return v;
 }
 
 struct Bfs {
@@ -231,10 +328,15 @@ struct StepIn {
     uint32_t end;    // one past the last entry the step covers
     uint32_t k;      // this group's entry
     uint32_t child;
-    bool gact;       // the group has an entry
-    bool act;        // the lane has a child
+    uint64_t groups; // lanes of the groups with an entry
+    uint64_t act;    // lanes with a child
     NodeData nd;
 };
+
+// Lanes of the first `n` groups of 8.
+__device__ __forceinline__ uint64_t group_lanes(uint32_t n) {
+    return n >= 8U ? ~0ULL : ((1ULL << (8U * n)) - 1ULL);
+}
 
 // Reads the entries [kb, min(kb + 8, tail)) of the queue and issues the loads of their children.
 template <bool kMixed, bool kMu0>
@@ -246,11 +348,11 @@ __device__ __forceinline__ StepIn fetch_step(const Lane& L, const CoopShared& sh
     x.kb = __builtin_amdgcn_readfirstlane(kb);
     x.end = __builtin_amdgcn_readfirstlane(min(kb + 8U, tail));
     x.k = kb + q;
-    x.gact = x.k < x.end;
-    const uint32_t packed = sh.queue[x.gact ? (x.k & (kQueueCap - 1U)) : kQueueCap];
+    x.groups = group_lanes(x.end - x.kb);
+    const uint32_t packed = sh.queue[x.k & (kQueueCap - 1U)];   // groups without an entry read a stale one
     x.child = (packed & kLinkMask) + j;
-    x.act = x.gact && j < (packed >> kLinkBits);
-    x.nd = load_node<kMixed, kMu0>(L, x.child, x.act);
+    x.act = x.groups & __builtin_amdgcn_ballot_w64(j < (packed >> kLinkBits));
+    x.nd = load_node<kMixed, kMu0>(L, x.child, __builtin_amdgcn_inverse_ballot_w64(x.act));
     return x;
 }
 
@@ -285,26 +387,28 @@ template <bool kMixed, bool kMu0>
 __device__ __forceinline__ bool bfs_step(const CoopArgs& a, const Lane& L, CoopShared& sh, const SlotTable& t,
                                          const StepIn& x, BfsState& b, Bfs& r) {
     const uint32_t ln = lane();
-    const uint32_t q = ln >> 3U, j = ln & 7U;
+    const uint32_t q = ln >> 3U;
     double p;
-    const int st = eval_node<kMixed, kMu0>(a.s, L, x.nd, x.child, x.act, &p);
-    r.tests += static_cast<uint32_t>(__popcll(__builtin_amdgcn_ballot_w64(x.act)));
-    r.count += static_cast<uint32_t>(__popcll(__builtin_amdgcn_ballot_w64(st == kAccept)));
+    const Verdict v = eval_node<kMixed, kMu0>(a.s, L, x.nd, x.child, x.act, sh.exp_table, &p);
+    r.tests += static_cast<uint32_t>(__popcll(x.act));
+    r.count += static_cast<uint32_t>(__popcll(v.accept));
     const double gsum = group_sum8(p);
-    const bool ex = st == kExpand;
-    const uint64_t em = __builtin_amdgcn_ballot_w64(ex);
+    const uint64_t em = v.expand;
     const uint32_t ne = static_cast<uint32_t>(__popcll(em));
     if (b.nslots + ne > t.dump || b.nslots + ne - b.flushed > kQueueCap) {
         return false;
     }
     // lane 8q (the one that writes group q's record) has rank_below(em) = the group's first slot
     const uint32_t slot = b.nslots + rank_below(em);
-    sh.queue[ex ? (slot & (kQueueCap - 1U)) : kQueueCap] = x.nd.m.y;
-    const bool gw = x.gact && j == 0;
-    const uint32_t gem = static_cast<uint32_t>((em >> (8U * q)) & 0xFFULL);
-    const uint32_t gi = gw ? (x.k & (kStageCap - 1U)) : kStageCap;
-    sh.stage_ms[gi] = gsum;
-    sh.stage_fx[gi] = (gem != 0 ? slot : kSlotNone) | (static_cast<uint32_t>(__popc(gem)) << 28U);
+    if (__builtin_amdgcn_inverse_ballot_w64(em)) {
+        sh.queue[slot & (kQueueCap - 1U)] = x.nd.m.y;
+    }
+    if (__builtin_amdgcn_inverse_ballot_w64(x.groups & 0x0101010101010101ULL)) {
+        const uint32_t gem = static_cast<uint32_t>(em >> (8U * q)) & 0xFFU;
+        const uint32_t gi = x.k & (kStageCap - 1U);
+        sh.stage_ms[gi] = gsum;
+        sh.stage_fx[gi] = (gem != 0 ? slot : kSlotNone) | (static_cast<uint32_t>(__popc(gem)) << 28U);
+    }
     // Levels that end inside this step: the level after each is the children of the groups before its
     // end.  A step can close two levels when the second was queued entirely before the step (the
     // last level of the traversal); an empty next level ends the traversal.  All of this is
@@ -318,8 +422,7 @@ __device__ __forceinline__ bool bfs_step(const CoopArgs& a, const Lane& L, CoopS
         if (!(kb < le && le <= end)) {
             break;
         }
-        const uint32_t gb = le - kb;
-        const uint64_t before = gb >= 8U ? ~0ULL : ((1ULL << (8U * gb)) - 1ULL);
+        const uint64_t before = group_lanes(le - kb);
         lev++;
         if (lev + 1 >= kMaxLevels + 4) {
             return false;
@@ -430,7 +533,8 @@ __device__ Bfs bfs(const CoopArgs& a, const Lane& L, uint32_t root_meta_y, CoopS
 // Resolves the draws of the active groups top-down through the slot table (one draw per group).
 // Returns the picked node in every lane of the group, kNone when the list had no positive mass.
 template <bool kMixed, bool kMu0>
-__device__ uint32_t navigate(const CoopArgs& a, const Lane& L, double rr, bool gact, uint64_t base, uint32_t* tests) {
+__device__ uint32_t navigate(const CoopArgs& a, const Lane& L, const double2* table, double rr, bool gact,
+                             uint64_t base, uint32_t* tests) {
     const SearchArgs& s = a.s;
     const uint32_t ln = lane();
     const uint32_t q = ln >> 3U, j = ln & 7U;
@@ -463,18 +567,14 @@ __device__ uint32_t navigate(const CoopArgs& a, const Lane& L, double rr, bool g
         const double mj_raw = at(tms, mact ? f + j : 0U);
         const double mj = mact ? mj_raw : 0.0;
         double p;
-        const int st = eval_node<kMixed, kMu0>(s, L, nd, fc + j, act, &p);
-        *tests += static_cast<uint32_t>(__popcll(__ballot(act)));
-        const uint64_t em = __ballot(act && st == kExpand);
+        const uint64_t actm = __builtin_amdgcn_ballot_w64(act);
+        const Verdict v = eval_node<kMixed, kMu0>(s, L, nd, fc + j, actm, table, &p);
+        *tests += static_cast<uint32_t>(__popcll(actm));
+        const uint64_t em = v.expand;
         const uint32_t gem = static_cast<uint32_t>((em >> g0) & 0xFFULL);
         const uint32_t rk = static_cast<uint32_t>(__popc(gem & ((1U << j) - 1U)));
         const double mexp = __shfl(mj, static_cast<int>(g0 + (rk & 7U)), kWave);
-        double mass = 0.0;
-        if (st == kAccept) {
-            mass = p;
-        } else if (st == kExpand) {
-            mass = mexp;
-        }
+        const double mass = __builtin_amdgcn_inverse_ballot_w64(em) ? mexp : p;   // p is 0 unless accepted
         const double cum = group_suffix8(mass);
         const double cum_next_raw = __shfl_down(cum, 1, kWave);
         const double cum_next = (j + 1 < 8) ? cum_next_raw : 0.0;
@@ -487,13 +587,13 @@ __device__ uint32_t navigate(const CoopArgs& a, const Lane& L, double rr, bool g
             jstar = __ffs(static_cast<int>(gpm)) - 1;
         }
         const uint32_t src_lane = g0 + static_cast<uint32_t>(jstar < 0 ? 0 : jstar);
-        const int stj = __shfl(st, static_cast<int>(src_lane), kWave);
+        const bool accj = ((v.accept >> src_lane) & 1ULL) != 0;
         const double before = __shfl(cum_next, static_cast<int>(src_lane), kWave);
         if (!done) {
             if (jstar < 0) {
                 done = true;
                 res = kNone;
-            } else if (stj == kAccept) {
+            } else if (accj) {
                 done = true;
                 res = fc + static_cast<uint32_t>(jstar);
             } else {
@@ -509,6 +609,13 @@ __device__ uint32_t navigate(const CoopArgs& a, const Lane& L, double rr, bool g
         }
     }
     return res;
+}
+
+// A sum below this goes to the per-lane search, which has the reference's fallbacks.  FP32-mixed
+// probabilities are FP32 numbers or exact ones, so only 0 does.
+template <bool kMixed>
+__device__ __forceinline__ constexpr double lowest_sum() {
+    return kMixed ? 5.0e-324 : kTiny;
 }
 
 struct ListResult {
@@ -532,7 +639,7 @@ __device__ ListResult list_of(const CoopArgs& a, const Lane& L, uint32_t root, C
     lr.tests = b.tests;
     lr.total = b.total;
     lr.count = b.count;
-    lr.overflow = b.overflow || (b.count > 0 && b.total == 0.0);
+    lr.overflow = b.overflow || (b.count > 0 && b.total < lowest_sum<kMixed>());
     return lr;
 }
 
@@ -546,7 +653,7 @@ enum : int { kDrawActive = 0, kDrawDone = 1, kDrawFailed = 2, kDrawSlow = 3, kDr
 // on its own.  A level that needs expansion, or whose Gaussian sum is 0 (the reference's fallbacks),
 // ends in kDrawSlow with (node, level) where the general per-lane traversal takes over.
 template <bool kMixed, bool kMu0>
-__device__ __forceinline__ int descend_fast(const SearchArgs& s, const Lane& L, uint32_t jd, int state, uint32_t& node,
+__device__ __forceinline__ int descend_fast(const SearchArgs& s, const Lane& L, const double2* table, uint32_t jd, int state, uint32_t& node,
                                             uint32_t& level, uint32_t& tests, unsigned long long& exec) {
     const uint32_t ln = lane();
     const uint32_t j = ln & 7U;
@@ -576,13 +683,14 @@ __device__ __forceinline__ int descend_fast(const SearchArgs& s, const Lane& L, 
         const bool act = act_g && j < nc;
         double p;
         const NodeData cd = load_node<kMixed, kMu0>(L, fc + j, act);
-        const int st = eval_node<kMixed, kMu0>(s, L, cd, fc + j, act, &p);
-        exec += static_cast<uint32_t>(__popcll(__builtin_amdgcn_ballot_w64(act)));
-        const uint32_t gexp = static_cast<uint32_t>((__builtin_amdgcn_ballot_w64(st == kExpand) >> g0) & 0xFFULL);
-        const uint32_t gacc = static_cast<uint32_t>((__builtin_amdgcn_ballot_w64(st == kAccept) >> g0) & 0xFFULL);
+        const uint64_t actm = __builtin_amdgcn_ballot_w64(act);
+        const Verdict v = eval_node<kMixed, kMu0>(s, L, cd, fc + j, actm, table, &p);
+        exec += static_cast<uint32_t>(__popcll(actm));
+        const uint32_t gexp = static_cast<uint32_t>(v.expand >> g0) & 0xFFU;
+        const uint32_t gacc = static_cast<uint32_t>(v.accept >> g0) & 0xFFU;
         const double gsum = __shfl(group_sum8(p), static_cast<int>(g0), kWave);
         if (act_g) {
-            if (gexp != 0 || (gacc != 0 && gsum == 0.0)) {
+            if (gexp != 0 || (gacc != 0 && gsum < lowest_sum<kMixed>())) {
                 state = kDrawSlow;
             } else {
                 tests += nc;
@@ -594,10 +702,9 @@ __device__ __forceinline__ int descend_fast(const SearchArgs& s, const Lane& L, 
         const bool pick = state == kDrawActive;
         const double r = pick ? draw_to_uniform(pick_draw(L.seed, L.local, L.step, jd, level), nextafter(gsum, gsum + 0.00001))
                               : 0.0;
-        const double pa = st == kAccept ? p : 0.0;
-        const double cum = group_suffix8(pa);
-        const uint32_t gcm = static_cast<uint32_t>((__builtin_amdgcn_ballot_w64(pa > 0.0 && cum >= r) >> g0) & 0xFFULL);
-        const uint32_t gpm = static_cast<uint32_t>((__builtin_amdgcn_ballot_w64(pa > 0.0) >> g0) & 0xFFULL);
+        const double cum = group_suffix8(p);
+        const uint32_t gcm = static_cast<uint32_t>((__builtin_amdgcn_ballot_w64(p > 0.0 && cum >= r) >> g0) & 0xFFULL);
+        const uint32_t gpm = static_cast<uint32_t>((__builtin_amdgcn_ballot_w64(p > 0.0) >> g0) & 0xFFULL);
         if (pick) {
             int jstar = -1;
             if (gcm != 0) {
@@ -635,6 +742,12 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8
     const uint64_t nw = *a.nwork;
     if (nw >= a.run_below) {
         return;   // the group walk takes this update
+    }
+    if (!kMixed) {
+        if (ln < 32) {
+            sh.exp_table[ln] = make_double2(kExpTable[ln][0], kExpTable[ln][1]);
+        }
+        __syncthreads();
     }
     const uint32_t step = *s.step;
     const uint32_t chunk = grab_size(nw, a.chunk);
@@ -702,10 +815,10 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8
             for (uint32_t j0 = 0; j0 < na; j0 += 8) {
                 const bool gact = j0 + q < na;
                 const double r = gact ? draw_to_uniform(pick_draw(L.seed, L.local, L.step, j0 + q, 1U), next1) : 0.0;
-                uint32_t node = navigate<kMixed, kMu0>(a, L, r, gact, base, &nav_tests);
+                uint32_t node = navigate<kMixed, kMu0>(a, L, sh.exp_table, r, gact, base, &nav_tests);
                 uint32_t level = 2, tests = l1.tests;
                 int state = !gact ? kDrawIdle : (node == kNone ? kDrawFailed : kDrawActive);
-                state = descend_fast<kMixed, kMu0>(s, L, j0 + q, state, node, level, tests, acc_exec);
+                state = descend_fast<kMixed, kMu0>(s, L, sh.exp_table, j0 + q, state, node, level, tests, acc_exec);
                 const bool lead = gact && j == 0;
                 const uint64_t sm = __builtin_amdgcn_ballot_w64(lead && state == kDrawSlow);
                 unsigned long long at0 = 0;
@@ -839,6 +952,8 @@ int launch_level1(rl_bh_ctx* c, const SearchArgs& sa, const uint32_t* work, cons
         k_level1<true, true><<<blocks, kWave, 0, s>>>(a);
     } else if (mixed) {
         k_level1<true, false><<<blocks, kWave, 0, s>>>(a);
+    } else if (mu0) {
+        k_level1<false, true><<<blocks, kWave, 0, s>>>(a);
     } else {
         k_level1<false, false><<<blocks, kWave, 0, s>>>(a);
     }

@@ -25,6 +25,7 @@ struct SearchArgs {
     const uint4* wrec[2];   // FP32 path: rec32 and meta side by side, two uint4 per node
     const uint2* meta[2];
     double theta;
+    double theta2;       // theta^2
     double scale64;      // -1 / sigma^2
     double mu;
     float theta2f;       // theta^2
