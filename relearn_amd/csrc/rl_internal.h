@@ -229,7 +229,9 @@ struct rl_bh_ctx {
     uint32_t coop_cap = 0;
     uint32_t coop_blocks = 0;        // persistent search waves: cus * waves_per_cu
     uint32_t cus = 0;
-    uint32_t waves_per_cu = 16;
+    // search waves per CU until tuned: what LDS and registers of the wave-per-source search allow (FP64 at
+    // 1M neurons: 12.3 ms at 16, 11.5 at 20); the group walk starts at 24
+    uint32_t waves_per_cu = 20;
     uint32_t search_chunk = 1;       // sources per work-queue grab of a search wave
     // group walk (the FP32-mixed search): per order position and type the active flags, their offsets,
     // the grouped source list, the (type, network) segments, and per wave the walk's tables

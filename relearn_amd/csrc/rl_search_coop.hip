@@ -10,7 +10,7 @@
 // Expanded nodes get a slot in a per-wave table: node, first expanded-child slot and count, and
 // the node's mass = total probability of the accepted candidates below it.  A group sums the
 // probabilities of its accepted children with a DPP butterfly; after the traversal the masses of
-// expanded children are pulled into their parents, deepest level first.  The mass of a node is the
+// expanded children are pulled into their parents, last slots first.  The mass of a node is the
 // span its subtree occupies in the reference's candidate list (descending Morton order = children
 // visited in descending octant order), so a draw r is resolved top-down
 // (ProbabilityPicker::pick_target, source/util/ProbabilityPicker.h:46-112): at each expanded node
@@ -37,11 +37,8 @@ namespace rl {
 namespace {
 
 constexpr int kWave = 64;
-constexpr uint32_t kQueueCap = 1024;   // LDS ring of queued / not yet flushed slots (power of two)
-constexpr uint32_t kStageCap = 256;    // LDS ring of slot records not yet flushed (power of two)
-constexpr uint32_t kFlushAt = 192;     // flush when this many processed slots are staged
 constexpr int kXcds = kCursorSlots;
-constexpr uint32_t kSlotNone = 0x0FFFFFFFU;
+constexpr uint32_t kFxSlot = 0x7FFU;   // slot bits of an fx entry
 
 struct CoopArgs {
     SearchArgs s;
@@ -49,10 +46,10 @@ struct CoopArgs {
     const uint64_t* nwork;        // device count of work; XCD segment x is [nwork x / 8, nwork (x + 1) / 8)
     unsigned long long* cursor;   // kXcds counters
     uint32_t chunk;               // sources taken from a segment per cursor increment
-    uint32_t* t_my;               // per wave: cap slots, packed child range of the slot's node
-    uint32_t* t_fexp;             // first expanded child slot | expanded-child count << 28
+    uint32_t* t_my;               // per wave: cap slots, of which those that left the LDS ring are used
+    uint32_t* t_fexp;
     double* t_mass;
-    uint32_t cap;
+    uint32_t cap;                 // at most 2,048: slots fit the 11 bits of fx
     uint32_t* overflow;
     unsigned long long* n_overflow;
     uint4* slow;                  // (slot, source, node, level) of descents for the per-lane kernel
@@ -60,16 +57,26 @@ struct CoopArgs {
     uint64_t run_below;           // the kernel returns at once when *nwork >= run_below
 };
 
-// Slot records are built in LDS during the traversal and copied to the wave's global slot table in
-// batches: a global store inside the step loop would make every step wait for the previous step's
-// stores (loads and stores share one wait counter).  The last entry of each ring takes the writes
-// of lanes with nothing to write.
+// The slot table of the source a wave works on: per expanded node its packed child range (which also makes
+// the table the traversal's queue), the slot of its first expanded child with their number, and its
+// mass.  LDS holds the last kRing slots at slot % kRing, the wave's part of the global table the ones
+// before: a source expands about 110 nodes at 1,000 neurons, 340 at 52,000, 550 at 1M and 640 at 4M
+// (theta 0.3), so few slots or none leave the ring, and those are the top of the tree.
+//
+// What bounds the search is the number of instructions of any kind that a wave issues one after another
+// (1.7 per cycle and SIMD at 5 waves, vector and scalar units 70% busy each), not one unit and not
+// memory.  With the whole table in global memory behind LDS staging rings, the level boundaries
+// tracked in every step and the reference's formulas inlined, a step took about 150 instructions and
+// the FP32-mixed kernel 96 VGPRs (5 waves per SIMD); now 105 and 80 (6 waves, 22 per CU by LDS).  1M
+// neurons: FP32-mixed 12.1 -> 8.8 ms, FP64 16.0 -> 11.5 ms.
+constexpr uint32_t kRing = 512;
+constexpr uint32_t kRingMask = kRing - 1U;
+template <bool kMixed>
 struct CoopShared {
-    uint32_t queue[kQueueCap + 1];     // packed child range (meta.y) of slot i at i % kQueueCap
-    uint32_t stage_fx[kStageCap + 1];  // first expanded child slot | count << 28 of slot i at i % kStageCap
-    double stage_ms[kStageCap + 1];    // probability mass of slot i at i % kStageCap
-    uint32_t lvl_start[kMaxLevels + 4];
-    double2 exp_table[32];             // 2^(i/32), first and second part (FP64 search only)
+    double ms[kRing];
+    double2 exp_table[kMixed ? 1 : 32]; // 2^(i/32), first and second part (FP64 search only)
+    uint32_t my[kRing];
+    uint16_t fx[kRing];                 // first expanded child's slot (if any) | expanded children << 11
 };
 
 __device__ __forceinline__ uint32_t lane() {
@@ -157,6 +164,25 @@ __device__ __forceinline__ NodeData load_node(const Lane& L, uint32_t node, bool
     return d;
 }
 
+struct ExactEval {
+    int st;
+    double p;
+};
+
+// The reference's own test and probability of a node, for the few that the test on squares leaves open.
+// Out of line: inlined into the traversal its divisions, square root and exponential cost the FP32-mixed
+// kernel a wave per SIMD (96 VGPRs instead of 80).
+__device__ __noinline__ ExactEval eval_reference(double theta, double mu, double scale64, double dx, double dy,
+                                                 double dz, double side, uint32_t count, bool leaf) {
+#pragma clang fp contract(off)
+    ExactEval e;
+    const double d = hypot3_exact(dx, dy, dz);
+    e.st = d == 0.0 ? kDiscard : (leaf || side < theta * d ? kAccept : kExpand);
+    const double exponent = ((d - mu) * (d - mu)) * scale64;
+    e.p = e.st == kAccept ? (exp(exponent) * 1.0) * static_cast<double>(count) : 0.0;
+    return e;
+}
+
 // 2^(i/32), i = 0..31, each as the nearest FP64 number and the nearest one to the rest.
 __constant__ const double kExpTable[32][2] = {
     { 0x1.0000000000000p+0, 0x0.0p+0 },
@@ -236,7 +262,7 @@ __device__ __forceinline__ double exp_gauss(double x, const double2* table) {
 // reference's; the Gaussian takes d^2 itself, which is rounded less than the square of the reference's
 // scaled hypot.  That hypot (three divisions and a square root, about 75 of the 210 vector
 // instructions of an FP64 step) and the library's exp made the FP64 search of 1M neurons 24.4 ms; with
-// squares and exp_gauss it takes 16.0 ms.
+// squares and exp_gauss it takes 16.0 ms (and 11.5 with the ring table below).
 template <bool kMixed, bool kMu0>
 __device__ __forceinline__ Verdict eval_node(const SearchArgs& a, const Lane& L, const NodeData& d, uint32_t node,
                                              uint64_t act, const double2* table, double* p_out) {
@@ -300,11 +326,10 @@ __device__ __forceinline__ Verdict eval_node(const SearchArgs& a, const Lane& L,
         int st = kDiscard;
         if (__builtin_amdgcn_inverse_ballot_w64(unsure)) {
             const bool leaf = (d.m.y >> kLinkBits) == 0;
-            const Eval e = kMixed ? eval_exact(a, L, node, 0, leaf) : eval_exact_rec(a, L, d.r64, leaf);
-            st = e.status;
-            if (st == kAccept) {
-                p = probability<false>(a, L, e, d.m.x, kGauss);
-            }
+            const double4 r = kMixed ? L.rec64[node] : d.r64;
+            const ExactEval e = eval_reference(a.theta, a.mu, a.scale64, r.x - L.px, r.y - L.py, r.z - L.pz, r.w, d.m.x, leaf);
+            st = e.st;
+            p = e.p;
         }
         v.accept |= __builtin_amdgcn_ballot_w64(st == kAccept);
         v.expand |= __builtin_amdgcn_ballot_w64(st == kExpand);
@@ -315,7 +340,7 @@ __device__ __forceinline__ Verdict eval_node(const SearchArgs& a, const Lane& L,
 
 struct Bfs {
     double total;
-    uint32_t count;
+    uint64_t accepted;   // not 0: the list has candidates
     uint32_t tests;
     bool overflow;
 };
@@ -338,9 +363,16 @@ __device__ __forceinline__ uint64_t group_lanes(uint32_t n) {
     return n >= 8U ? ~0ULL : ((1ULL << (8U * n)) - 1ULL);
 }
 
+struct SlotTable {   // the global part, indexed by slot
+    uint32_t* my;
+    uint32_t* fx;
+    double* ms;
+    uint32_t dump;   // one past the last slot
+};
+
 // Reads the entries [kb, min(kb + 8, tail)) of the queue and issues the loads of their children.
 template <bool kMixed, bool kMu0>
-__device__ __forceinline__ StepIn fetch_step(const Lane& L, const CoopShared& sh, uint32_t kb, uint32_t tail) {
+__device__ __forceinline__ StepIn fetch_step(const Lane& L, const CoopShared<kMixed>& sh, uint32_t kb, uint32_t tail) {
     const uint32_t ln = lane();
     const uint32_t q = ln >> 3U, j = ln & 7U;
     StepIn x;
@@ -349,109 +381,68 @@ __device__ __forceinline__ StepIn fetch_step(const Lane& L, const CoopShared& sh
     x.end = __builtin_amdgcn_readfirstlane(min(kb + 8U, tail));
     x.k = kb + q;
     x.groups = group_lanes(x.end - x.kb);
-    const uint32_t packed = sh.queue[x.k & (kQueueCap - 1U)];   // groups without an entry read a stale one
+    const uint32_t packed = sh.my[x.k & kRingMask];   // groups without an entry read a stale one
     x.child = (packed & kLinkMask) + j;
     x.act = x.groups & __builtin_amdgcn_ballot_w64(j < (packed >> kLinkBits));
     x.nd = load_node<kMixed, kMu0>(L, x.child, __builtin_amdgcn_inverse_ballot_w64(x.act));
     return x;
 }
 
-struct SlotTable {
-    uint32_t* my;
-    uint32_t* fx;
-    double* ms;
-    uint32_t dump;   // last slot: takes the stores of lanes with nothing to store
-};
-
 struct BfsState {
     uint32_t nslots;   // queue tail = slots allocated
-    uint32_t lvl_end;  // one past the last slot of the level being processed
-    uint32_t lev;      // that level
-    uint32_t flushed;  // slots below this are in the global table
+    uint32_t out;      // slots below left the ring for the global table
 };
 
-// Copies the records of slots [from, to) from the LDS rings to the global slot table.
-__device__ __forceinline__ void flush_slots(const SlotTable& t, const CoopShared& sh, uint32_t from, uint32_t to) {
-    for (uint32_t sl = from + lane(); sl < to; sl += kWave) {
-        at(t.my, sl) = sh.queue[sl & (kQueueCap - 1U)];
-        at(t.fx, sl) = sh.stage_fx[sl & (kStageCap - 1U)];
-        at(t.ms, sl) = sh.stage_ms[sl & (kStageCap - 1U)];
-    }
-}
-
 // Tests the children of one step's entries, sums the accepted probabilities per group, appends the
-// expanded children to the queue and records the entries' masses.  Entries of two consecutive levels
-// can share a step; the level boundary is tracked for the upward mass pass.  Returns false when the
-// slot table, the queue or the level table would overflow.
+// expanded children to the table and records the entries' masses.  Ends the traversal when the table would
+// overflow, or the ring with slots not yet processed.
 template <bool kMixed, bool kMu0>
-__device__ __forceinline__ bool bfs_step(const CoopArgs& a, const Lane& L, CoopShared& sh, const SlotTable& t,
+__device__ __forceinline__ void bfs_step(const CoopArgs& a, const Lane& L, CoopShared<kMixed>& sh, const SlotTable& t,
                                          const StepIn& x, BfsState& b, Bfs& r) {
     const uint32_t ln = lane();
     const uint32_t q = ln >> 3U;
     double p;
     const Verdict v = eval_node<kMixed, kMu0>(a.s, L, x.nd, x.child, x.act, sh.exp_table, &p);
     r.tests += static_cast<uint32_t>(__popcll(x.act));
-    r.count += static_cast<uint32_t>(__popcll(v.accept));
+    r.accepted |= v.accept;
     const double gsum = group_sum8(p);
     const uint64_t em = v.expand;
-    const uint32_t ne = static_cast<uint32_t>(__popcll(em));
-    if (b.nslots + ne > t.dump || b.nslots + ne - b.flushed > kQueueCap) {
-        return false;
-    }
+    const uint32_t ns = __builtin_amdgcn_readfirstlane(b.nslots);
+    const uint32_t tail = ns + static_cast<uint32_t>(__popcll(em));
     // lane 8q (the one that writes group q's record) has rank_below(em) = the group's first slot
-    const uint32_t slot = b.nslots + rank_below(em);
-    if (__builtin_amdgcn_inverse_ballot_w64(em)) {
-        sh.queue[slot & (kQueueCap - 1U)] = x.nd.m.y;
-    }
+    const uint32_t slot = ns + rank_below(em);
     if (__builtin_amdgcn_inverse_ballot_w64(x.groups & 0x0101010101010101ULL)) {
         const uint32_t gem = static_cast<uint32_t>(em >> (8U * q)) & 0xFFU;
-        const uint32_t gi = x.k & (kStageCap - 1U);
-        sh.stage_ms[gi] = gsum;
-        sh.stage_fx[gi] = (gem != 0 ? slot : kSlotNone) | (static_cast<uint32_t>(__popc(gem)) << 28U);
+        const uint32_t gi = x.k & kRingMask;
+        sh.ms[gi] = gsum;
+        sh.fx[gi] = static_cast<uint16_t>(slot | (static_cast<uint32_t>(__popc(gem)) << 11U));
     }
-    // Levels that end inside this step: the level after each is the children of the groups before its
-    // end.  A step can close two levels when the second was queued entirely before the step (the
-    // last level of the traversal); an empty next level ends the traversal.  All of this is
-    // wave-uniform scalar work.
-    const uint32_t kb = __builtin_amdgcn_readfirstlane(x.kb);
-    const uint32_t end = __builtin_amdgcn_readfirstlane(x.end);
-    const uint32_t ns = __builtin_amdgcn_readfirstlane(b.nslots);
-    uint32_t le = __builtin_amdgcn_readfirstlane(b.lvl_end);
-    uint32_t lev = __builtin_amdgcn_readfirstlane(b.lev);
-    for (int pass = 0; pass < 2; pass++) {
-        if (!(kb < le && le <= end)) {
-            break;
+    if (tail > b.out + kRing) {
+        // 64 processed slots leave the ring (a step adds at most 64)
+        if (tail > t.dump || b.out + kWave > x.end) {
+            r.overflow = true;
+            b.nslots = 0;   // ends the traversal
+            return;
         }
-        const uint64_t before = group_lanes(le - kb);
-        lev++;
-        if (lev + 1 >= kMaxLevels + 4) {
-            return false;
-        }
-        if (ln == 0) {
-            sh.lvl_start[lev] = le;
-        }
-        const uint32_t next_end = ns + static_cast<uint32_t>(__popcll(em & before));
-        if (next_end == le) {
-            break;
-        }
-        le = next_end;
+        const uint32_t sl = b.out + ln;
+        at(t.my, sl) = sh.my[sl & kRingMask];
+        at(t.fx, sl) = sh.fx[sl & kRingMask];
+        at(t.ms, sl) = sh.ms[sl & kRingMask];
+        b.out += kWave;
     }
-    b.lvl_end = le;
-    b.lev = lev;
-    b.nslots = ns + ne;
-    if (x.end - b.flushed >= kFlushAt) {
-        flush_slots(t, sh, b.flushed, x.end);
-        b.flushed = __builtin_amdgcn_readfirstlane(x.end);
+    if (__builtin_amdgcn_inverse_ballot_w64(em)) {
+        sh.my[slot & kRingMask] = x.nd.m.y;
     }
-    return true;
+    b.nslots = tail;
 }
 
-// Breadth-first traversal below `root` (inner, with vacant dendrites) filling the slot table at `base`.
-// The queue is consumed 8 entries per step across level boundaries; the next step's child records are
+// Breadth-first traversal below `root` (inner, with vacant dendrites) filling the slot table.  The queue
+// is consumed 8 entries per step across level boundaries; the next step's child records are
 // loaded before the current step is evaluated (two alternating step buffers, so no registers are
-// copied).
+// copied).  *out gets the number of slots in the global table.
 template <bool kMixed, bool kMu0>
-__device__ Bfs bfs(const CoopArgs& a, const Lane& L, uint32_t root_meta_y, CoopShared& sh, uint64_t base) {
+__device__ Bfs bfs(const CoopArgs& a, const Lane& L, uint32_t root_meta_y, CoopShared<kMixed>& sh, uint64_t base,
+                   uint32_t* out) {
     const uint32_t ln = lane();
     Bfs r{ 0.0, 0, 0, false };
     SlotTable t;
@@ -460,14 +451,12 @@ __device__ Bfs bfs(const CoopArgs& a, const Lane& L, uint32_t root_meta_y, CoopS
     t.ms = a.t_mass + base;
     t.dump = a.cap - 1;
     if (ln == 0) {
-        sh.queue[0] = root_meta_y;
-        sh.lvl_start[0] = 0;
+        sh.my[0] = root_meta_y;
     }
     __syncthreads();
-    BfsState b{ 1U, 1U, 0U, 0U };
+    BfsState b{ 1U, 0U };
     StepIn xa = fetch_step<kMixed, kMu0>(L, sh, 0U, 1U);
-    // Wait for the first step's data here, so that the loop header carries no pending load and the
-    // stores of the previous step are never waited for.
+    // Wait for the first step's data here, so that the loop header carries no pending load.
     if (kMixed) {
         __asm__ volatile("" ::"v"(xa.nd.m.x), "v"(xa.nd.m.y), "v"(xa.nd.r32.x), "v"(xa.nd.r32.y), "v"(xa.nd.r32.z),
                          "v"(xa.nd.r32.w));
@@ -478,63 +467,77 @@ __device__ Bfs bfs(const CoopArgs& a, const Lane& L, uint32_t root_meta_y, CoopS
     while (true) {
         StepIn xb = fetch_step<kMixed, kMu0>(L, sh, xa.end, b.nslots);
         __builtin_amdgcn_sched_barrier(0);   // keep the prefetch ahead of this step's work
-        if (!bfs_step<kMixed, kMu0>(a, L, sh, t, xa, b, r)) {
-            r.overflow = true;
-            return r;
-        }
+        bfs_step<kMixed, kMu0>(a, L, sh, t, xa, b, r);
         if (xb.kb >= b.nslots) {
             break;
         }
         xa = fetch_step<kMixed, kMu0>(L, sh, xb.end, b.nslots);
         __builtin_amdgcn_sched_barrier(0);
-        if (!bfs_step<kMixed, kMu0>(a, L, sh, t, xb, b, r)) {
-            r.overflow = true;
-            return r;
-        }
+        bfs_step<kMixed, kMu0>(a, L, sh, t, xb, b, r);
         if (xa.kb >= b.nslots) {
             break;
         }
     }
-    const uint32_t lev = b.lev;
-    flush_slots(t, sh, b.flushed, b.nslots);
+    if (r.overflow) {
+        return r;
+    }
     __syncthreads();
-    // pull the masses of expanded children into their parents, deepest parents first
-    for (int lv = static_cast<int>(lev) - 2; lv >= 0; lv--) {
-        const uint32_t sb = sh.lvl_start[lv], se = sh.lvl_start[lv + 1];
-        for (uint32_t i0 = sb; i0 < se; i0 += kWave) {
-            const uint32_t sl = i0 + ln;
-            if (sl < se) {
-                const uint32_t fx = at(t.fx, sl);
-                const uint32_t ne = fx >> 28U;
-                const uint32_t f = fx & kSlotNone;
-                if (ne != 0 && f + ne <= t.dump) {
-                    double m8[8];
+    // Pull the masses of expanded children into their parents, last slots first, up to 64 at a time: the
+    // slots [lo, hi) above the last one of the 64 with a child below hi.  All their children lie at or beyond
+    // hi and have their final masses; slot hi - 1 always is one of them, since children follow parents.
+    *out = b.out;
+    uint32_t hi = __builtin_amdgcn_readfirstlane(b.nslots);
+    while (hi > 0) {
+        const uint32_t first = hi > kWave ? hi - kWave : 0U;
+        const uint32_t sl = first + ln;
+        const bool in_lds = first >= b.out;   // then the children are too
+        uint32_t fx = 0;
+        if (sl < hi) {
+            fx = in_lds || sl >= b.out ? sh.fx[sl & kRingMask] : at(t.fx, sl);
+        }
+        const uint32_t f = fx & kFxSlot;
+        const uint32_t ne = fx >> 11U;
+        const uint64_t open = __builtin_amdgcn_ballot_w64(ne != 0 && f < hi);
+        const uint32_t lo = open == 0 ? first : first + kWave - static_cast<uint32_t>(__builtin_clzll(open));
+        if (sl >= lo && ne != 0) {
+            double m8[8];
+            if (in_lds) {
 #pragma unroll
-                    for (uint32_t c = 0; c < 8; c++) {
-                        m8[c] = at(t.ms, f + (c < ne ? c : 0U));
-                    }
-                    double sum = 0.0;
-#pragma unroll
-                    for (uint32_t c = 0; c < 8; c++) {
-                        if (c < ne) {
-                            sum += m8[c];
-                        }
-                    }
-                    at(t.ms, sl) += sum;
+                for (uint32_t c = 0; c < 8; c++) {
+                    m8[c] = sh.ms[(f + c) & kRingMask];
                 }
+            } else {
+#pragma unroll
+                for (uint32_t c = 0; c < 8; c++) {
+                    const uint32_t k = f + (c < ne ? c : 0U);
+                    m8[c] = k >= b.out ? sh.ms[k & kRingMask] : at(t.ms, k);
+                }
+            }
+            double sum = 0.0;
+#pragma unroll
+            for (uint32_t c = 0; c < 8; c++) {
+                if (c < ne) {
+                    sum += m8[c];
+                }
+            }
+            if (in_lds || sl >= b.out) {
+                sh.ms[sl & kRingMask] += sum;
+            } else {
+                at(t.ms, sl) += sum;
             }
         }
         __syncthreads();
+        hi = lo;
     }
-    r.total = t.ms[0];
+    r.total = b.out == 0 ? sh.ms[0] : t.ms[0];
     return r;
 }
 
 // Resolves the draws of the active groups top-down through the slot table (one draw per group).
 // Returns the picked node in every lane of the group, kNone when the list had no positive mass.
 template <bool kMixed, bool kMu0>
-__device__ uint32_t navigate(const CoopArgs& a, const Lane& L, const double2* table, double rr, bool gact,
-                             uint64_t base, uint32_t* tests) {
+__device__ uint32_t navigate(const CoopArgs& a, const Lane& L, const CoopShared<kMixed>& sh, uint32_t out, double rr,
+                             bool gact, uint64_t base, uint32_t* tests) {
     const SearchArgs& s = a.s;
     const uint32_t ln = lane();
     const uint32_t q = ln >> 3U, j = ln & 7U;
@@ -550,25 +553,35 @@ __device__ uint32_t navigate(const CoopArgs& a, const Lane& L, const double2* ta
             break;
         }
         // slot < cap always holds: it only advances to a checked child slot
-        uint32_t fx = at(tfx, slot);
-        uint32_t my = at(tmy, slot);
+        uint32_t fx, my;
+        if (__builtin_amdgcn_ballot_w64(slot < out) == 0) {
+            fx = sh.fx[slot & kRingMask];
+            my = sh.my[slot & kRingMask];
+        } else {
+            fx = slot >= out ? sh.fx[slot & kRingMask] : at(tfx, slot);
+            my = slot >= out ? sh.my[slot & kRingMask] : at(tmy, slot);
+        }
         if (done) {
             fx = 0;
             my = 0;
         }
         const uint32_t fc = my & kLinkMask;
         const uint32_t nc = my >> kLinkBits;
-        const uint32_t f = fx & kSlotNone;
-        const uint32_t nexp = fx >> 28U;
+        const uint32_t f = fx & kFxSlot;
+        const uint32_t nexp = fx >> 11U;
         const bool act = !done && j < nc;
         // the children and the masses of the expanded ones, loaded together
         const NodeData nd = load_node<kMixed, kMu0>(L, fc + j, act);
-        const bool mact = !done && j < nexp && f != kSlotNone && f + j < a.cap;
-        const double mj_raw = at(tms, mact ? f + j : 0U);
-        const double mj = mact ? mj_raw : 0.0;
+        const uint32_t mk = j < nexp ? f + j : slot;
+        double mj;
+        if (__builtin_amdgcn_ballot_w64(mk < out) == 0) {
+            mj = sh.ms[mk & kRingMask];
+        } else {
+            mj = mk >= out ? sh.ms[mk & kRingMask] : at(tms, mk);
+        }
         double p;
         const uint64_t actm = __builtin_amdgcn_ballot_w64(act);
-        const Verdict v = eval_node<kMixed, kMu0>(s, L, nd, fc + j, actm, table, &p);
+        const Verdict v = eval_node<kMixed, kMu0>(s, L, nd, fc + j, actm, sh.exp_table, &p);
         *tests += static_cast<uint32_t>(__popcll(actm));
         const uint64_t em = v.expand;
         const uint32_t gem = static_cast<uint32_t>((em >> g0) & 0xFFULL);
@@ -599,7 +612,7 @@ __device__ uint32_t navigate(const CoopArgs& a, const Lane& L, const double2* ta
             } else {
                 rr = rr - before;
                 const uint32_t next = f + static_cast<uint32_t>(__popc(gem & ((1U << jstar) - 1U)));
-                if (f == kSlotNone || next >= a.cap - 1) {
+                if (nexp == 0 || next >= a.cap - 1) {
                     done = true;
                     res = kNone;
                 } else {
@@ -620,8 +633,9 @@ __device__ __forceinline__ constexpr double lowest_sum() {
 
 struct ListResult {
     double total;
-    uint32_t count;
+    bool any;        // the list has candidates
     uint32_t tests;
+    uint32_t out;    // slots in the global table
     bool overflow;   // slot table overflow or a Gaussian sum of 0: the per-lane kernel redoes the source
 };
 
@@ -629,17 +643,17 @@ struct ListResult {
 // reference's fallbacks (Kernel::create_probability_interval, Kernel.h:109-126), which the per-lane
 // kernel implements, so the source is handed over.
 template <bool kMixed, bool kMu0>
-__device__ ListResult list_of(const CoopArgs& a, const Lane& L, uint32_t root, CoopShared& sh, uint64_t base) {
-    ListResult lr{ 0.0, 0, 0, false };
+__device__ ListResult list_of(const CoopArgs& a, const Lane& L, uint32_t root, CoopShared<kMixed>& sh, uint64_t base) {
+    ListResult lr{ 0.0, false, 0, 0, false };
     const uint2 mr = L.meta[root];
     if (mr.x == 0) {
         return lr;
     }
-    const Bfs b = bfs<kMixed, kMu0>(a, L, mr.y, sh, base);
+    const Bfs b = bfs<kMixed, kMu0>(a, L, mr.y, sh, base, &lr.out);
     lr.tests = b.tests;
     lr.total = b.total;
-    lr.count = b.count;
-    lr.overflow = b.overflow || (b.count > 0 && b.total < lowest_sum<kMixed>());
+    lr.any = b.accepted != 0;
+    lr.overflow = b.overflow || (lr.any && b.total < lowest_sum<kMixed>());
     return lr;
 }
 
@@ -726,13 +740,11 @@ __device__ __forceinline__ int descend_fast(const SearchArgs& s, const Lane& L, 
 // One wave per source builds the candidate list of the root once (BarnesHutBase::find_target_neuron
 // re-derives it for every axon, BarnesHutBase.h:223-255), resolves the source's level-1 draws against
 // it 8 at a time, and continues each draw's descent in its group.  Results go to slot_target; descents
-// that need the general traversal are queued for the per-lane kernel.  Both instances are held to 5
-// waves per SIMD (at most 96 VGPRs): the FP64 one needs 98 otherwise; to fit, it spills one 64-bit
-// value (stored once, reloaded once per source, never in the step loop), and measures 5% faster at 20
-// waves per CU than at 4 waves per SIMD.
+// that need the general traversal are queued for the per-lane kernel.  Registers: FP32-mixed is held to 6
+// waves per SIMD (80 VGPRs; 11.0 against 11.3 ms per 1M-neuron update at 5), FP64 to 5 (96).
 template <bool kMixed, bool kMu0>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8))) k_level1(CoopArgs a) {
-    __shared__ CoopShared sh;
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kMixed ? 6 : 5, 8))) k_level1(CoopArgs a) {
+    __shared__ CoopShared<kMixed> sh;
     const SearchArgs& s = a.s;
     const uint32_t ln = lane();
     const uint32_t q = ln >> 3U, j = ln & 7U;
@@ -805,7 +817,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8
                 a.overflow[k] = src;
                 s.found[src] = kOverflowMark;
             }
-        } else if (l1.count == 0) {
+        } else if (!l1.any) {
             if (ln == 0) {
                 s.slot_tests[slot0] = l1.tests;   // slot_target[slot0] stays kNone: one failed search
             }
@@ -815,7 +827,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5, 8
             for (uint32_t j0 = 0; j0 < na; j0 += 8) {
                 const bool gact = j0 + q < na;
                 const double r = gact ? draw_to_uniform(pick_draw(L.seed, L.local, L.step, j0 + q, 1U), next1) : 0.0;
-                uint32_t node = navigate<kMixed, kMu0>(a, L, sh.exp_table, r, gact, base, &nav_tests);
+                uint32_t node = navigate<kMixed, kMu0>(a, L, sh, l1.out, r, gact, base, &nav_tests);
                 uint32_t level = 2, tests = l1.tests;
                 int state = !gact ? kDrawIdle : (node == kNone ? kDrawFailed : kDrawActive);
                 state = descend_fast<kMixed, kMu0>(s, L, sh.exp_table, j0 + q, state, node, level, tests, acc_exec);

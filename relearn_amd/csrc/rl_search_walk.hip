@@ -872,8 +872,8 @@ int launch_search_walk(rl_bh_ctx* c, const SearchArgs& sa) {
     if (timed) RL_HIP(c, hipEventRecord(c->ev2, s));
     if (a.run_from > 0) {
         // the wave-per-source kernel over the same lists (sources of each type in Morton order), at the
-        // setting its tuning picks for updates below the threshold (20 waves per CU, 8 sources per grab)
-        RL_TRY(launch_level1(c, sa, c->walk_list, n_active, a.run_from, c->cus * 20U, 8U));
+        // setting its tuning picks for updates below the threshold (22 waves per CU, 8 sources per grab)
+        RL_TRY(launch_level1(c, sa, c->walk_list, n_active, a.run_from, c->cus * 22U, 8U));
     }
     // the counting instantiation is a separate kernel: the counters change the register allocation of the walk
     const bool count = (c->cfg.flags & RL_FLAG_COUNT_WALK) != 0;
