@@ -80,4 +80,43 @@ __device__ __forceinline__ double draw_to_uniform(uint32_t k, double next) {
     return numerator / 4294967296.0 * (next - 0.0) + 0.0;
 }
 
+// Kernels that visit every neuron or group and end by adding to a device counter: blocks of 1,024
+// threads, two per CU of a 256-CU GPU, so that few atomics meet at the counter.
+constexpr int kCountThreads = 1024;
+constexpr unsigned kCountBlocks = 512;
+
+inline unsigned count_blocks(uint64_t n) {
+    const uint64_t b = (n + kCountThreads - 1) / kCountThreads;
+    return static_cast<unsigned>(b == 0 ? 1 : (b < kCountBlocks ? b : kCountBlocks));
+}
+
+// Sums each of the N values over a block of kCountThreads threads; thread 0 gets the totals.
+template <int N>
+__device__ __forceinline__ void block_totals(unsigned long long (&v)[N]) {
+    __shared__ unsigned long long part[N][kCountThreads / 64];
+    const uint32_t ln = threadIdx.x & 63U;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            v[k] += __shfl_xor(v[k], o, 64);
+        }
+        if (ln == 0) {
+            part[k][threadIdx.x / 64U] = v[k];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 64U) {
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            unsigned long long t = ln < kCountThreads / 64U ? part[k][ln] : 0;
+#pragma unroll
+            for (int o = 8; o > 0; o >>= 1) {
+                t += __shfl_xor(t, o, 64);
+            }
+            v[k] = t;
+        }
+    }
+}
+
 }  // namespace rl

@@ -18,7 +18,7 @@ constexpr uint32_t kNoTarget = 0xFFFFFFFFU;
 constexpr int kDrawsPerPass = 8;             // draws resolved per pick traversal
 constexpr unsigned kStreamBlocks = 2048;     // grid of the grid-stride kernels sized on the device
 constexpr int kCursorSlots = 8;              // work cursors of the persistent search waves, one per XCD
-constexpr int kCursorStride = 16;            // 64-bit words between cursors: a 128-byte line each
+constexpr int kCursorStride = 16;            // 64-bit words between cursors: a 128-byte line each (word 1: tests)
 constexpr uint32_t kMaxWavesPerCu = 24;      // slot tables are allocated for this many search waves per CU
 
 // Device counters of one update (rl_bh_ctx::counters), zeroed at the start of every search and read

@@ -490,6 +490,7 @@ __global__ void k_search_reset(uint64_t n, const uint64_t* __restrict__ slot_tot
     }
     if (t0 < kCursorSlots) {
         cursor[t0 * kCursorStride] = 0;
+        cursor[t0 * kCursorStride + 1] = 0;
     }
 }
 
@@ -547,12 +548,18 @@ __global__ void __launch_bounds__(kBlock) k_candidates(SearchArgs a, const uint3
     counts[t] = static_cast<uint32_t>(v.count);
 }
 
-__global__ void k_collect(unsigned long long* __restrict__ counters, const uint64_t* __restrict__ slots,
+__global__ void k_collect(unsigned long long* __restrict__ counters, const unsigned long long* __restrict__ cursor,
+                          const uint64_t* __restrict__ slots,
                           const uint64_t* __restrict__ requests, const uint64_t* __restrict__ active) {
     if (threadIdx.x == 0) {
         counters[kCtrSlots] = *slots;
         counters[kCtrRequests] = *requests;
         counters[kCtrActive] = *active;
+        unsigned long long exec = 0;
+        for (int x = 0; x < kCursorSlots; x++) {
+            exec += cursor[x * kCursorStride + 1];
+        }
+        counters[kCtrTestsExec] += exec;
     }
 }
 
@@ -726,7 +733,7 @@ int enqueue_search(rl_bh_ctx* c) {
     k_emit_requests<<<grid_for(n), kBlock, 0, s>>>(n, c->found, c->req_off, c->slot_off, c->slot_target, c->signal,
                                                     c->req_target, c->req_source, c->req_signal, c->req_j);
     RL_HIP(c, hipGetLastError());
-    k_collect<<<1, 64, 0, s>>>(c->counters, c->slot_off + n, c->req_off + n, n_active);
+    k_collect<<<1, 64, 0, s>>>(c->counters, c->coop_cursor, c->slot_off + n, c->req_off + n, n_active);
     RL_HIP(c, hipGetLastError());
     return RL_OK;
 }

@@ -853,26 +853,18 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kMix
         __syncthreads();
     }
     if (ln == 0 && acc_exec != 0) {
-        atomicAdd(&s.counters[kCtrTestsExec], acc_exec);
+        // beside the wave's XCD's cursor; k_collect adds the eight up
+        atomicAdd(&a.cursor[(blockIdx.x % kXcds) * kCursorStride + 1], acc_exec);
     }
-}
-
-__device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        v += __shfl_xor(v, o, kWave);
-    }
-    return v;
 }
 
 // Per source, in axon order: a search that fails ends the source's searches (find_target_neurons,
 // BarnesHutBase.h:283-289).  Counts the searches, the successful ones and the reference's tests.
 // Neurons in index order, grid-stride, so that neighbouring lanes read neighbouring slots (the work
 // list is in Morton order, whose slots are scattered).  The totals are summed per block and added
-// with one atomic per block: atomics of every wave on the same two counters serialise (they took
-// 6 ms at 16M).
-__global__ void __launch_bounds__(256) k_finalize(SearchArgs s) {
-    __shared__ unsigned long long part[2][256 / kWave];
+// with one atomic per block and counter: same-address atomics pass one after another.  At 1M neurons the
+// kernel took 58 us with 2,048 blocks, 21 us now.
+__global__ void __launch_bounds__(kCountThreads) k_finalize(SearchArgs s) {
     unsigned long long ref = 0, searched_n = 0;
     const bool over = s.counters[kCtrOverCap] != 0;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
@@ -902,24 +894,11 @@ __global__ void __launch_bounds__(256) k_finalize(SearchArgs s) {
         s.searched[src] = searched;
         searched_n += searched;
     }
-    ref = wave_sum(ref);
-    searched_n = wave_sum(searched_n);
-    const uint32_t wv = threadIdx.x / kWave;
-    if ((threadIdx.x & (kWave - 1)) == 0) {
-        part[0][wv] = ref;
-        part[1][wv] = searched_n;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long r = 0, sn = 0;
-        for (uint32_t k = 0; k < 256 / kWave; k++) {
-            r += part[0][k];
-            sn += part[1][k];
-        }
-        if (sn != 0) {
-            atomicAdd(&s.counters[kCtrTestsRef], r);
-            atomicAdd(&s.counters[kCtrSearches], sn);
-        }
+    unsigned long long sum[2] = { ref, searched_n };
+    block_totals(sum);
+    if (threadIdx.x == 0 && sum[1] != 0) {
+        atomicAdd(&s.counters[kCtrTestsRef], sum[0]);
+        atomicAdd(&s.counters[kCtrSearches], sum[1]);
     }
 }
 
@@ -974,8 +953,7 @@ int launch_level1(rl_bh_ctx* c, const SearchArgs& sa, const uint32_t* work, cons
 }
 
 int launch_finalize(rl_bh_ctx* c, const SearchArgs& sa) {
-    const uint64_t n = std::max<uint64_t>(c->n, 1);
-    k_finalize<<<static_cast<unsigned>(std::min<uint64_t>((n + 255) / 256, kStreamBlocks)), 256, 0, c->stream>>>(sa);
+    k_finalize<<<count_blocks(c->n), kCountThreads, 0, c->stream>>>(sa);
     RL_HIP(c, hipGetLastError());
     return RL_OK;
 }
