@@ -25,11 +25,9 @@ inline unsigned grid_for(uint64_t n, int block = kBlock) {
     return static_cast<unsigned>(g == 0 ? 1 : g);
 }
 
-__device__ __forceinline__ double growth_curve(double current, double eta, double epsilon) {
+// The growth curve of one element type; branch-free, so that the three types interleave.  table: kExpTable.
+__device__ __forceinline__ double growth_curve(double current, double eta, double epsilon, const double2* table) {
 #pragma clang fp contract(off)
-    if (eta == epsilon) {
-        return current == eta ? 0.0 : -1.0;
-    }
     constexpr double factor = 1.6651092223153955127063292897904020952611777045288814583336582344;
     constexpr double factor_inv = 1.0 / factor;
     const double xi = (eta + epsilon) * 0.5;
@@ -37,7 +35,10 @@ __device__ __forceinline__ double growth_curve(double current, double eta, doubl
     const double difference = current - xi;
     const double quotient = difference / zeta;
     const double product = quotient * quotient;
-    return (2.0 * exp(-product)) - 1.0;
+    // exp is 0 below -745.2; the clamp keeps the exponent arithmetic in range and lets a NaN through
+    const double x = product > 800.0 ? -800.0 : -product;
+    const double curve = (2.0 * exp_gauss(x, table)) - 1.0;
+    return eta == epsilon ? (current == eta ? 0.0 : -1.0) : curve;
 }
 
 // Normal(mean, stddev) from two Philox words (tag 3) by the Box-Muller transform in FP32 on 24-bit
@@ -88,13 +89,23 @@ struct StepArgs {
     double tau_inv;
 };
 
-// A neuron that fired adds the weight of each of its out-pairs to the target's input of the next
-// step (integer atomics: the sums do not depend on their order).  Few neurons fire per step, so
+// Element i of an array that the whole launch shares: scalar base, 32-bit byte offset (at most 2^28
+// neurons of 8 bytes).
+template <typename T>
+__device__ __forceinline__ T& at(T* base, uint32_t i) {
+    return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + i * static_cast<uint32_t>(sizeof(T)));
+}
+
+template <typename T>
+__device__ __forceinline__ const T& at(const T* base, uint32_t i) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + i * static_cast<uint32_t>(sizeof(T)));
+}
+
+// A neuron that fired adds the weight of each of its out-pairs [e0, e1) to the target's input of the
+// next step (integer atomics: the sums do not depend on their order).  Few neurons fire per step, so
 // this replaces a gather over every in-edge of every neuron.
 // Pairs are read four at a time, so that their loads overlap.
-__device__ __forceinline__ void push_out_pairs(const StepArgs& a, uint64_t i) {
-    const uint64_t e0 = a.out_off[i];
-    const uint64_t e1 = a.out_off[i + 1];
+__device__ __forceinline__ void push_out_pairs(const StepArgs& a, uint64_t e0, uint64_t e1) {
     for (uint64_t e = e0; e < e1; e += 4) {
         uint32_t t[4];
         int32_t w[4];
@@ -113,53 +124,88 @@ __device__ __forceinline__ void push_out_pairs(const StepArgs& a, uint64_t i) {
     }
 }
 
+// One step of one neuron per lane.
+//
+// At 1M neurons the kernel moves its 106 bytes per neuron at 4.2 TB/s, 0.8 of what a device copy
+// reaches; below about 500,000 neurons (one round of waves) the time is a wave's own chain of loads and
+// about 545 vector instructions.  They were about 650, with 64-bit addresses, the library's exp in three
+// divergent branches, vector keys for Philox and a loop over the substeps.  1M neurons without synaptic
+// input: 28.0 -> 25.5 us; 2M with it: 62 -> 57 us.  Fewer resident waves, so that rounds overlap, are
+// slower (6 blocks per CU instead of 8: +2%, 4: +6%).
+// kSub: substeps of a step (the reference's 10) unrolled, or 0 for p.h of any number.
+template <uint32_t kSub>
 __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
 #pragma clang fp contract(off)
-    const uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
-    if (i >= a.n) {
-        return;
-    }
-    const uint64_t n = a.n;
+    __shared__ double2 table[32];
+    const uint32_t n = static_cast<uint32_t>(a.n);
+    const uint32_t lane_i = blockIdx.x * static_cast<uint32_t>(kBlock) + threadIdx.x;
+    const bool in = lane_i < n;
+    const uint32_t i = in ? lane_i : n - 1U;
     const rl_step_params& p = a.p;
     // every per-neuron load first, so that they are in flight together instead of one round trip
     // after another
-    const uint8_t en = a.enabled[i];
-    const uint8_t fprev = a.fired_prev[i];
-    const uint32_t g = a.net_of != nullptr ? a.net_of[i] : 0U;
-    double xv = a.x[i];
-    double uv = a.u[i];
-    double c = a.ca[i];
-    const double tgt = a.target_ca != nullptr ? a.target_ca[i] : a.target_value;
-    const double dl[3] = { a.delta[i], a.delta[n + i], a.delta[2 * n + i] };
-    const double caller_input = p.input_mode == 0 ? a.input[i] : 0.0;
+    const uint8_t en = at(a.enabled, i);
+    const uint8_t fprev = at(a.fired_prev, i);
+    const uint32_t g = a.net_of != nullptr ? at(a.net_of, i) : 0U;
+    double xv = at(a.x, i);
+    double uv = at(a.u, i);
+    double c = at(a.ca, i);
+    const double tgt = a.target_ca != nullptr ? at(a.target_ca, i) : a.target_value;
+    double* const delta[3] = { a.delta, a.delta + a.n, a.delta + 2 * a.n };
+    const double dl[3] = { at(delta[0], i), at(delta[1], i), at(delta[2], i) };
+    double input = p.input_mode == 0 ? at(a.input, i) : 0.0;
     const bool synaptic = a.acc_cur != nullptr;
-    const int32_t syn = synaptic ? a.acc_cur[i] : 0;
+    const int32_t syn = synaptic ? at(a.acc_cur, i) : 0;
+    if (threadIdx.x < 32) {
+        table[threadIdx.x] = make_double2(kExpTable[threadIdx.x][0], kExpTable[threadIdx.x][1]);
+    }
+    __syncthreads();
+    if (!in) {
+        return;
+    }
     if (en == 0) {
-        a.fired[i] = fprev;  // the step leaves a disabled neuron's status as it was
+        at(a.fired, i) = fprev;  // the step leaves a disabled neuron's status as it was
         if (synaptic) {
-            a.acc_cur[i] = 0;
+            at(a.acc_cur, i) = 0;
             if (fprev != 0) {
-                push_out_pairs(a, i);
+                push_out_pairs(a, a.out_off[i], a.out_off[i + 1]);
             }
         }
         return;
     }
-    const uint32_t step = a.step_base != nullptr ? *a.step_base + a.step : a.step;
-    double input = p.input_mode == 0 ? caller_input
-                                     : normal_input(a.net_seed[g], static_cast<uint32_t>(i - a.net_off[g]), step,
-                                                    p.input_mean, p.input_stddev);
+    if (p.input_mode != 0) {
+        const uint32_t step = a.step_base != nullptr ? *a.step_base + a.step : a.step;
+        // neurons of one network are neighbours: one pass per network among the wave's lanes, nearly
+        // always one, with the network's seed and first neuron in scalar registers
+        bool todo = true;
+        while (todo) {
+            const uint32_t g0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(g)));
+            if (g == g0) {
+                const uint64_t seed = a.net_seed[g0];
+                const uint32_t first = static_cast<uint32_t>(a.net_off[g0]);
+                const uint32_t s0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(seed)));
+                const uint32_t s1 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(seed >> 32U)));
+                input = normal_input(s0 | static_cast<uint64_t>(s1) << 32U, i - first, step, p.input_mean, p.input_stddev);
+                todo = false;
+            }
+        }
+    }
     if (synaptic) {
         // SynapticEquallyWeightedActivityInputCPU::update_local_input: the weights of the in-edges
         // whose source fired in the previous step, times the conductance.  The sum was pushed by those
         // sources; it is an integer, which the reference's FP64 accumulation of integer weights
         // yields exactly.  CombinedActivityInputCPU adds it to the background input.
         input = input + static_cast<double>(syn) * a.conductance;
-        a.acc_cur[i] = 0;
+        if (syn != 0) {
+            at(a.acc_cur, i) = 0;
+        }
     }
     const double scale = a.scale;
     const double ab = p.a * p.b;
-    uint8_t spiked = 0;
-    for (uint32_t s = 0; s < p.h; s++) {
+    const uint32_t h = kSub != 0 ? kSub : p.h;
+    bool spiked = false;
+#pragma unroll
+    for (uint32_t s = 0; s < h; s++) {
         const double x_increase = (p.k1 * xv * xv) + (p.k2 * xv) + p.k3 - uv + input;
         const double u_increase = (ab * xv) - (p.a * uv);
         xv += x_increase * scale;
@@ -167,28 +213,44 @@ __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
         if (xv >= p.v_spike) {
             xv = p.c;
             uv += p.d;
-            spiked = 1;
+            spiked = true;
             break;
         }
     }
-    a.fired[i] = spiked;
-    a.x[i] = xv;
-    a.u[i] = uv;
-    if (synaptic && spiked != 0) {
-        push_out_pairs(a, i);
+    at(a.fired, i) = spiked ? 1 : 0;
+    at(a.x, i) = xv;
+    at(a.u, i) = uv;
+    const bool push = synaptic && spiked;
+    uint64_t e0 = 0, e1 = 0;   // read here, used at the end
+    if (push) {
+        e0 = a.out_off[i];
+        e1 = a.out_off[i + 1];
     }
     const double tau_inv = a.tau_inv;
-    const double local_beta = p.beta_ca * static_cast<double>(spiked == 1);
-    for (uint32_t s = 0; s < p.h; s++) {
+    const double local_beta = p.beta_ca * (spiked ? 1.0 : 0.0);
+#pragma unroll
+    for (uint32_t s = 0; s < h; s++) {
         c += scale * (c * tau_inv + local_beta);
     }
-    a.ca[i] = c;
+    at(a.ca, i) = c;
+#pragma unroll
     for (int t = 0; t < 3; t++) {
-        const double eta = a.min_ca != nullptr ? a.min_ca[t * n + i] : p.eta[t];
+        const double eta = a.min_ca != nullptr ? at(a.min_ca + t * a.n, i) : p.eta[t];
         const double clamped_target = tgt < eta ? eta : tgt;  // std::max(target, eta)
-        const double dz = growth_curve(c, eta, clamped_target);
+        const double dz = growth_curve(c, eta, clamped_target, table);
         const double nu = a.net_nu != nullptr ? a.net_nu[3 * static_cast<uint64_t>(g) + t] : p.nu[t];
-        a.delta[t * n + i] = dl[t] + dz * nu;
+        at(delta[t], i) = dl[t] + dz * nu;
+    }
+    if (push) {
+        push_out_pairs(a, e0, e1);
+    }
+}
+
+void launch_step(const StepArgs& a, hipStream_t s) {
+    if (a.p.h == 10) {
+        k_step<10><<<grid_for(a.n), kBlock, 0, s>>>(a);
+    } else {
+        k_step<0><<<grid_for(a.n), kBlock, 0, s>>>(a);
     }
 }
 
@@ -455,7 +517,7 @@ int neurons_step(rl_bh_ctx* c, uint32_t step, const double* input) {
     }
     StepArgs a = step_args(c);
     a.step = step;
-    k_step<<<grid_for(n), kBlock, 0, c->stream>>>(a);
+    launch_step(a, c->stream);
     RL_HIP(c, hipGetLastError());
     s.parity ^= 1;
     s.fired = s.fired_buf[s.parity];
@@ -501,7 +563,7 @@ int enqueue_neuron_steps(rl_bh_ctx* c, uint32_t steps) {
             a.acc_cur = c->net.acc[k & 1U];
             a.acc_next = c->net.acc[(k + 1) & 1U];
         }
-        k_step<<<grid_for(c->n), kBlock, 0, c->stream>>>(a);
+        launch_step(a, c->stream);
         RL_HIP(c, hipGetLastError());
     }
     if ((steps & 1U) != 0) {
