@@ -13,6 +13,13 @@ constexpr int kScanItems = 16;                      // counts per thread
 constexpr uint64_t kScanTile = kScanBlock * kScanItems;
 constexpr int kTopBlock = 1024;                     // the single block that scans the tile sums
 constexpr int kTopItems = 8;
+// Launches of a scan.  A small kernel costs 5-8 us from launch to launch whatever it does, in a captured
+// graph too, so up to kOneBlockCounts counts are scanned by one block (two passes of 16,384), and while
+// the tile sums are few (kOwnPrefixTiles) every block of the last kernel adds up those before its own
+// instead of waiting for a kernel that does.  With three launches at every size the scans of a
+// 1,000-neuron update took 15 of its 48 launches.
+constexpr uint64_t kOneBlockCounts = 32768;
+constexpr uint64_t kOwnPrefixTiles = 1024;
 constexpr int kWave = 64;
 
 // Thread t of tile b owns counts [b * 4096 + 16 t, + 16); counts at or beyond n read as 0.
@@ -65,20 +72,68 @@ __device__ __forceinline__ uint64_t block_exclusive(uint64_t x, uint64_t* wave_s
     return off + inc - x;
 }
 
-__global__ void __launch_bounds__(kScanBlock) k_scan_reduce(const uint32_t* __restrict__ in, uint64_t n,
-                                                            uint64_t* __restrict__ part) {
-    __shared__ uint64_t ws[kScanBlock / kWave];
-    uint32_t v[kScanItems];
-    load_counts(in, blockIdx.x * kScanTile + threadIdx.x * static_cast<uint64_t>(kScanItems), n, v);
+// Writes the exclusive prefix sums `run`, run + v[0], ... of a thread's counts.
+__device__ __forceinline__ void store_prefix(uint64_t* __restrict__ out, uint64_t first, uint64_t n, uint64_t run,
+                                             const uint32_t (&v)[kScanItems]) {
+    uint64_t o[kScanItems];
+#pragma unroll
+    for (int k = 0; k < kScanItems; k++) {
+        o[k] = run;
+        run += v[k];
+    }
+    if (first + kScanItems <= n) {
+        ulonglong2* p = reinterpret_cast<ulonglong2*>(out + first);
+#pragma unroll
+        for (int k = 0; k < kScanItems / 2; k++) {
+            p[k] = make_ulonglong2(o[2 * k], o[2 * k + 1]);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++) {
+            if (first + k < n) {
+                out[first + k] = o[k];
+            }
+        }
+    }
+}
+
+__device__ __forceinline__ uint64_t sum_counts(const uint32_t (&v)[kScanItems]) {
     uint64_t s = 0;
 #pragma unroll
     for (int k = 0; k < kScanItems; k++) {
         s += v[k];
     }
+    return s;
+}
+
+__global__ void __launch_bounds__(kScanBlock) k_scan_reduce(const uint32_t* __restrict__ in, uint64_t n,
+                                                            uint64_t* __restrict__ part) {
+    __shared__ uint64_t ws[kScanBlock / kWave];
+    uint32_t v[kScanItems];
+    load_counts(in, blockIdx.x * kScanTile + threadIdx.x * static_cast<uint64_t>(kScanItems), n, v);
     uint64_t tot = 0;
-    (void)block_exclusive<kScanBlock>(s, ws, &tot);
+    (void)block_exclusive<kScanBlock>(sum_counts(v), ws, &tot);
     if (threadIdx.x == 0) {
         part[blockIdx.x] = tot;
+    }
+}
+
+// One block scans everything.
+__global__ void __launch_bounds__(kTopBlock) k_scan_one(const uint32_t* __restrict__ in, uint64_t n,
+                                                        uint64_t* __restrict__ out) {
+    __shared__ uint64_t ws[kTopBlock / kWave];
+    uint64_t carry = 0;
+    for (uint64_t base = 0; base < n; base += static_cast<uint64_t>(kTopBlock) * kScanItems) {
+        const uint64_t first = base + threadIdx.x * static_cast<uint64_t>(kScanItems);
+        uint32_t v[kScanItems];
+        load_counts(in, first, n, v);
+        uint64_t tot = 0;
+        const uint64_t run = carry + block_exclusive<kTopBlock>(sum_counts(v), ws, &tot);
+        store_prefix(out, first, n, run, v);
+        carry += tot;
+    }
+    if (threadIdx.x == 0) {
+        out[n] = carry;
     }
 }
 
@@ -112,38 +167,32 @@ __global__ void __launch_bounds__(kTopBlock) k_scan_top(uint64_t* __restrict__ p
     }
 }
 
+// kOwnPrefix: part holds the tiles' sums, and the block adds up the ones before its own (at most
+// kOwnPrefixTiles); the last block writes the total.  Else part holds their prefix sums.
+template <bool kOwnPrefix>
 __global__ void __launch_bounds__(kScanBlock) k_scan_down(const uint32_t* __restrict__ in, uint64_t n,
                                                           const uint64_t* __restrict__ part, uint64_t* __restrict__ out) {
     __shared__ uint64_t ws[kScanBlock / kWave];
     const uint64_t first = blockIdx.x * kScanTile + threadIdx.x * static_cast<uint64_t>(kScanItems);
     uint32_t v[kScanItems];
     load_counts(in, first, n, v);
-    uint64_t s = 0;
+    uint64_t before = 0;
+    if (kOwnPrefix) {
+        uint64_t mine = 0;
 #pragma unroll
-    for (int k = 0; k < kScanItems; k++) {
-        s += v[k];
+        for (uint64_t k = 0; k < kOwnPrefixTiles / kScanBlock; k++) {
+            const uint64_t t = k * kScanBlock + threadIdx.x;
+            mine += t < blockIdx.x ? part[t] : 0;
+        }
+        (void)block_exclusive<kScanBlock>(mine, ws, &before);
+    } else {
+        before = part[blockIdx.x];
     }
     uint64_t tot = 0;
-    uint64_t run = part[blockIdx.x] + block_exclusive<kScanBlock>(s, ws, &tot);
-    uint64_t o[kScanItems];
-#pragma unroll
-    for (int k = 0; k < kScanItems; k++) {
-        o[k] = run;
-        run += v[k];
-    }
-    if (first + kScanItems <= n) {
-        ulonglong2* p = reinterpret_cast<ulonglong2*>(out + first);
-#pragma unroll
-        for (int k = 0; k < kScanItems / 2; k++) {
-            p[k] = make_ulonglong2(o[2 * k], o[2 * k + 1]);
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < kScanItems; k++) {
-            if (first + k < n) {
-                out[first + k] = o[k];
-            }
-        }
+    const uint64_t run = before + block_exclusive<kScanBlock>(sum_counts(v), ws, &tot);
+    store_prefix(out, first, n, run, v);
+    if (kOwnPrefix && blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) {
+        out[n] = before + tot;
     }
 }
 
@@ -173,18 +222,24 @@ uint64_t scan_scratch_entries(uint64_t n) {
 }
 
 hipError_t scan_counts_on(hipStream_t s, const uint32_t* in, uint64_t n, uint64_t* out, uint64_t* part) {
+    if (n <= kOneBlockCounts) {
+        k_scan_one<<<1, kTopBlock, 0, s>>>(in, n, out);
+        return hipGetLastError();
+    }
     const uint64_t tiles = (n + kScanTile - 1) / kScanTile;
-    if (tiles > 0) {
-        k_scan_reduce<<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, n, part);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) {
-            return e;
-        }
+    k_scan_reduce<<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, n, part);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        return e;
+    }
+    if (tiles <= kOwnPrefixTiles) {
+        k_scan_down<true><<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, n, part, out);
+        return hipGetLastError();
     }
     k_scan_top<<<1, kTopBlock, 0, s>>>(part, tiles, out + n);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && tiles > 0) {
-        k_scan_down<<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, n, part, out);
+    e = hipGetLastError();
+    if (e == hipSuccess) {
+        k_scan_down<false><<<static_cast<unsigned>(tiles), kScanBlock, 0, s>>>(in, n, part, out);
         e = hipGetLastError();
     }
     return e;

@@ -382,28 +382,31 @@ __device__ __forceinline__ uint32_t quant_side2(double side, double scale) {
     return __float_as_uint(static_cast<float>(sq * sq));
 }
 
-// One thread per (node, dendrite type) of a level: the type's count and FP64 centroid of an inner node
-// from its children (children loaded together, then summed in child order 0..7), clamped to the cell
-// box, and its fixed-point record.
-__global__ void k_upward_level(uint64_t first, uint64_t last, const double* __restrict__ nbox,
-                               double4* __restrict__ rec0, double4* __restrict__ rec1, uint2* __restrict__ meta0,
-                               uint2* __restrict__ meta1, uint4* __restrict__ q0, uint4* __restrict__ q1,
-                               const uint32_t* __restrict__ node_net, QuantArgs qa) {
+struct UpwardArgs {
+    const double* nbox;
+    double4* rec0;
+    double4* rec1;
+    uint2* meta0;
+    uint2* meta1;
+    uint4* q0;
+    uint4* q1;
+    const uint32_t* node_net;
+    QuantArgs qa;
+};
+
+// Node i, dendrite type s: the type's count and FP64 centroid of an inner node from its children
+// (children loaded together, then summed in child order 0..7), clamped to the cell box, and its
+// fixed-point record.
+__device__ __forceinline__ void upward_node(const UpwardArgs& u, uint64_t i, int s) {
 #pragma clang fp contract(off)
-    const uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
-    const uint64_t i = first + (t >> 1U);
-    const int s = static_cast<int>(t & 1U);
-    if (i >= last) {
-        return;
-    }
-    const uint32_t packed = meta0[i].y;
+    const uint32_t packed = u.meta0[i].y;
     const uint32_t nc = packed >> kLinkBits;
     if (nc == 0) {
         return;  // leaves keep the neuron position (Cell::set_neuron_position)
     }
     const uint32_t fc = packed & kLinkMask;
-    double4* rec = s == 0 ? rec0 : rec1;
-    uint2* meta = s == 0 ? meta0 : meta1;
+    double4* rec = s == 0 ? u.rec0 : u.rec1;
+    uint2* meta = s == 0 ? u.meta0 : u.meta1;
     uint32_t cn[8];
     double4 cp[8];
 #pragma unroll
@@ -432,7 +435,7 @@ __global__ void k_upward_level(uint64_t first, uint64_t last, const double* __re
     if (total != 0) {
         const double w = static_cast<double>(total);
         double qx = ax / w, qy = ay / w, qz = az / w;
-        const double* b = nbox + 6 * i;
+        const double* b = u.nbox + 6 * i;
         qx = qx < b[0] ? b[0] : (b[3] < qx ? b[3] : qx);
         qy = qy < b[1] ? b[1] : (b[4] < qy ? b[4] : qy);
         qz = qz < b[2] ? b[2] : (b[5] < qz ? b[5] : qz);
@@ -445,13 +448,43 @@ __global__ void k_upward_level(uint64_t first, uint64_t last, const double* __re
         r.z = 0.0;
     }
     rec[i] = r;
-    if (qa.enabled) {
-        uint4* q = s == 0 ? q0 : q1;
-        const uint32_t g = node_net[i];
-        const double* lo = qa.net_box + 6 * static_cast<uint64_t>(g);
-        const double sc = qa.net_scale[g];
+    if (u.qa.enabled) {
+        uint4* q = s == 0 ? u.q0 : u.q1;
+        const uint32_t g = u.node_net[i];
+        const double* lo = u.qa.net_box + 6 * static_cast<uint64_t>(g);
+        const double sc = u.qa.net_scale[g];
         q[i] = make_uint4(quantize(r.x, lo[0], sc), quantize(r.y, lo[1], sc), quantize(r.z, lo[2], sc),
                           quant_side2(r.w, sc));
+    }
+}
+
+// One thread per (node, dendrite type) of a level.
+__global__ void k_upward_level(uint64_t first, uint64_t last, UpwardArgs u) {
+    const uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
+    const uint64_t i = first + (t >> 1U);
+    if (i < last) {
+        upward_node(u, i, static_cast<int>(t & 1U));
+    }
+}
+
+// Consecutive levels of few nodes by one block, deepest first.  A launch costs 5-8 us and a pass of the
+// block over 512 nodes about 2 us, so levels of up to kFewNodes go together: at 1,000 neurons the
+// seven launches of the upward pass become two, at 1M fourteen become seven.
+constexpr uint64_t kFewNodes = 1024;
+constexpr int kFewThreads = 1024;
+
+struct LevelRange {
+    uint32_t count;                      // levels, deepest first
+    uint32_t start[kMaxLevels + 1];      // node range [start, end) of each
+    uint32_t end[kMaxLevels + 1];
+};
+
+__global__ void __launch_bounds__(kFewThreads) k_upward_few(LevelRange r, UpwardArgs u) {
+    for (uint32_t l = 0; l < r.count; l++) {
+        for (uint32_t t = threadIdx.x; t < 2U * (r.end[l] - r.start[l]); t += kFewThreads) {
+            upward_node(u, r.start[l] + (t >> 1U), static_cast<int>(t & 1U));
+        }
+        __syncthreads();
     }
 }
 
@@ -767,15 +800,29 @@ int prepare_tree(rl_bh_ctx* c) {
     k_leaf_fill<<<grid_for(c->n), kBlock, 0, s>>>(c->n, c->leaf_of, c->enabled, c->vac[1], c->vac[2], t.meta[0],
                                                    t.meta[1]);
     RL_HIP(c, hipGetLastError());
-    const QuantArgs qa = quant_args(c);
-    for (int l = static_cast<int>(t.depth) - 1; l >= 0; l--) {
-        const uint64_t first = t.level_start[l], last = t.level_start[l + 1];
-        if (last <= first) {
-            continue;
+    UpwardArgs u{};
+    u.nbox = t.box;
+    u.rec0 = t.rec64[0];
+    u.rec1 = t.rec64[1];
+    u.meta0 = t.meta[0];
+    u.meta1 = t.meta[1];
+    u.q0 = t.rec32[0];
+    u.q1 = t.rec32[1];
+    u.node_net = t.node_net;
+    u.qa = quant_args(c);
+    for (int l = static_cast<int>(t.depth) - 1; l >= 0;) {
+        LevelRange few{};
+        for (; l >= 0 && t.level_start[l + 1] - t.level_start[l] <= kFewNodes; l--) {
+            few.start[few.count] = static_cast<uint32_t>(t.level_start[l]);
+            few.end[few.count++] = static_cast<uint32_t>(t.level_start[l + 1]);
         }
-        k_upward_level<<<grid_for(2 * (last - first)), kBlock, 0, s>>>(first, last, t.box, t.rec64[0], t.rec64[1],
-                                                                        t.meta[0], t.meta[1], t.rec32[0], t.rec32[1],
-                                                                        t.node_net, qa);
+        if (few.count > 0) {
+            k_upward_few<<<1, kFewThreads, 0, s>>>(few, u);
+        } else {
+            const uint64_t first = t.level_start[l], last = t.level_start[l + 1];
+            k_upward_level<<<grid_for(2 * (last - first)), kBlock, 0, s>>>(first, last, u);
+            l--;
+        }
         RL_HIP(c, hipGetLastError());
     }
     return RL_OK;
