@@ -1085,7 +1085,10 @@ int rl_bh_graph_create(rl_bh_ctx* c, uint32_t steps, uint64_t max_vacant_axons) 
     if (status == RL_OK) status = enqueue_commit(c, nullptr);
     if (status == RL_OK) status = enqueue_net_append(c);
     // the next period's steps push over the pairs as this period left them
-    if (status == RL_OK && c->neurons.ready && c->neurons.p.synaptic_input != 0) status = enqueue_syn_sync(c, 0);
+    if (status == RL_OK && c->neurons.ready && c->neurons.p.synaptic_input != 0) {
+        status = enqueue_out_lists(c);
+        if (status == RL_OK) status = enqueue_syn_push(c, 0);
+    }
     c->capturing = false;
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(s, &g);
@@ -1139,9 +1142,9 @@ int rl_bh_graph_launch(rl_bh_ctx* c, uint32_t first_step, uint32_t update, rl_bh
         RL_HIP(c, hipEventRecord(c->ev0, s));
     }
     RL_HIP(c, hipGraphLaunch(c->graph_exec, s));
-    if (synaptic) {
-        c->net.syn_valid = true;   // the period ends by rebuilding the pushes over its pairs
-    }
+    // with synaptic input the period ends by rebuilding lists and pushes over its pairs
+    c->net.out_valid = synaptic;
+    c->net.syn_valid = synaptic;
     c->prepared = false;
     c->searched_valid = false;
     c->nreq = 0;

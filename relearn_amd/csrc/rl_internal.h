@@ -88,27 +88,28 @@ struct NetGraph {
     uint32_t* src = nullptr;       // cap
     int32_t* w = nullptr;          // cap
     uint64_t* off2 = nullptr;      // n + 1: merge buffers
-    uint32_t* src2 = nullptr;
+    uint32_t* src2 = nullptr;      // in scratch
     int32_t* w2 = nullptr;
     uint32_t* ncnt = nullptr;      // n: synapses appended per target, then merged entries per target
     uint64_t* npre = nullptr;      // n + 1: prefix sums of ncnt
-    uint32_t* ocnt = nullptr;      // n: out-entries per source of a deletion phase
-    uint64_t* ooff = nullptr;      // n + 1
-    uint2* olist = nullptr;        // cap: (entry, target) of each out-entry, grouped by source
-    // Synaptic input by push: the non-zero pairs grouped by source, and per step parity the summed
-    // weights that the neurons which fired pushed to their targets for the next step.
+    // The non-zero pairs grouped by source: what a source that fires pushes (synaptic input), and the
+    // pairs among which a source deletes axons.
     uint64_t* out_off = nullptr;   // n + 1
-    uint32_t* out_cnt = nullptr;   // n: zero between builds
-    uint32_t* out_tgt = nullptr;   // cap
-    int32_t* out_w = nullptr;      // cap
+    uint2* out_pair = nullptr;     // cap: target, weight
+    uint32_t* out_entry = nullptr; // cap: the pair's entry in src and w
+    uint32_t* bin_cnt = nullptr;   // grouping: pairs per (bin of sources, block), and their prefix sums
+    uint64_t* bin_off = nullptr;
+    uint4* scratch = nullptr;      // cap: the pairs in bins (source, target, weight, entry), or src2 and w2
+    // per step parity the summed weights that the neurons which fired pushed to their targets for the next step
     int32_t* acc[2] = { nullptr, nullptr };  // n each
     uint64_t cap = 0;
     // host: an upper bound of the graph's entries, exact after a call that synchronised with the device
     // and raised by each replay without stats by the most synapses a period can append
     uint64_t entries_bound = 0;
     bool ready = false;
-    // acc[parity] holds the pushes of fired_buf[parity] over the current pairs, acc[parity ^ 1] is
-    // zero, and the out-edge lists match the graph
+    bool out_valid = false;   // the lists by source match the graph
+    // out_valid, acc[parity] holds the pushes of fired_buf[parity] over the current pairs, and
+    // acc[parity ^ 1] is zero
     bool syn_valid = false;
 };
 
@@ -376,8 +377,9 @@ int enqueue_net_append(rl_bh_ctx* c);   // appends the accepted requests of the 
 int enqueue_net_delete(rl_bh_ctx* c, int type);  // deletes the synapses of the type's shrunken elements
 int net_append(rl_bh_ctx* c);           // eager: grows the capacity if needed, then appends
 int net_append_retry(rl_bh_ctx* c);     // after a captured append over capacity: grow, then append
-int enqueue_syn_sync(rl_bh_ctx* c, int parity);  // out-edge lists from the graph, acc from fired_buf[parity]
-int syn_prepare(rl_bh_ctx* c);          // enqueue_syn_sync at the current parity unless syn_valid
+int enqueue_out_lists(rl_bh_ctx* c);    // the lists by source from the graph
+int enqueue_syn_push(rl_bh_ctx* c, int parity);  // acc from fired_buf[parity] and the lists by source
+int syn_prepare(rl_bh_ctx* c);          // both, at the current parity, unless they are valid
 void net_free(rl_bh_ctx* c);
 
 }  // namespace rl

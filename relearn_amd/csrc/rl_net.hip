@@ -165,48 +165,277 @@ __global__ void k_net_offsets(uint64_t n, const uint64_t* __restrict__ noff, uin
     }
 }
 
+// ---------------------------------------------------------------- pairs by source
+
+// The pairs grouped by source come from a counting sort in two levels, without global atomics.  Sources
+// fall into bins of 2^shift.  k_out_bins<false> counts the pairs of each block of targets per bin; after
+// a prefix sum over (bin, block), k_out_bins<true> writes them there as 16-byte records, so that a
+// block's records of one bin are consecutive.  k_out_sort then sorts a bin's records by source in LDS
+// and writes them in order.  One count and one scatter over all sources, each with one global atomic per
+// pair, were bound by the atomics (26 G/s) and by 4-byte writes to lines that had left L2 by the next
+// write: 608 + 1,256 us for 16M pairs of 2M sources, against 83 + 258 + 144 us and 10 us of prefix sum
+// (1.2 GB moved); axon deletions needed 666 us more for lists of their own.  9 periods of 300,001
+// neurons in all: 235 -> 71 us.
+//
+// More bins cost k_out_bins partly written lines (a block's open line per bin, 32 x bins x 128 B in an
+// XCD's L2), fewer cost k_out_sort: k_out_bins<true> + k_out_sort took 199 + 551 us with 512 bins,
+// 239 + 333 with 2,048 and 258 + 222 with 4,096 when k_out_sort scattered to memory; with the records
+// sorted in LDS 258 + 144 us with 4,096 bins and 286 + 188 with 8,192.  One block per CU: 512 blocks do
+// not gain.
+constexpr uint64_t kOutBlocks = 256;
+constexpr uint32_t kOutThreads = 1024;
+constexpr uint32_t kOutBins = 4096;        // below; more once a bin's counters would not fit into 64 KB of LDS
+constexpr uint32_t kOutMinShift = 8;
+constexpr uint32_t kOutMaxShift = 14;
+constexpr uint32_t kOutHeld = 8;           // records per thread that k_out_sort holds
+constexpr uint32_t kOutStaged = kOutHeld * kOutThreads;
+constexpr uint32_t kOutStageShift = 12;    // staging area and counters share the LDS up to this bin size
+// Small graphs are sorted by one block in one launch: the four launches of the larger sort take about
+// 5 us each, and the one block 21 us for 8,000 pairs (1,000 neurons) and more in proportion, so that
+// by the capacity's bound of 32,768 it is at worst some 50 us behind.
+constexpr uint64_t kOutOneSources = 2048;
+constexpr uint64_t kOutOnePairs = 32768;
+
+uint32_t out_shift(uint64_t n) {
+    uint32_t shift = kOutMinShift;
+    while (shift < kOutMaxShift && (n >> shift) >= kOutBins) {
+        shift++;
+    }
+    return shift;
+}
+
+uint64_t out_bins(uint64_t n) {
+    return (n + (1ULL << out_shift(n)) - 1) >> out_shift(n);
+}
+
+uint64_t out_blocks(uint64_t n) {
+    return std::min<uint64_t>(kOutBlocks, (n + kOutThreads - 1) / kOutThreads);
+}
+
+// f(entry, target, source, weight) for the non-zero pairs of targets [t0, min(t0 + 64, t1)): the wave reads the
+// entries in order; a lane finds its entry's target by bisection over the 64 offsets.
+template <typename F>
+__device__ __forceinline__ void wave_pairs(uint64_t t0, uint64_t t1, const uint64_t* __restrict__ off,
+                                           const uint32_t* __restrict__ src, const int32_t* __restrict__ w, F f) {
+    const uint32_t lane = threadIdx.x & 63U;
+    const uint64_t mine = off[t0 + lane < t1 ? t0 + lane : t1];
+    const uint64_t lo = __shfl(static_cast<unsigned long long>(mine), 0);
+    const uint32_t rel = static_cast<uint32_t>(mine - lo);
+    const uint32_t m = static_cast<uint32_t>(off[t0 + 64 < t1 ? t0 + 64 : t1] - lo);
+    for (uint32_t j0 = 0; j0 < m; j0 += 64) {
+        const uint32_t j = j0 + lane;
+        const bool in = j < m;
+        const uint32_t s = in ? src[lo + j] : 0U;
+        const int32_t we = in ? w[lo + j] : 0;
+        uint32_t k = 0;   // the last target whose list starts at or before j
+#pragma unroll
+        for (uint32_t step = 32; step != 0; step >>= 1) {
+            const uint32_t start = __shfl(rel, static_cast<int>(k + step));
+            k += start <= j ? step : 0U;
+        }
+        if (we != 0) {
+            f(lo + j, t0 + k, s, we);
+        }
+    }
+}
+
+// Block b takes targets [b per, (b + 1) per).  kWrite: records to the bin's place, else counts per bin.
+template <bool kWrite>
+__global__ void __launch_bounds__(kOutThreads) k_out_bins(uint64_t n, uint64_t per, uint32_t shift, uint32_t bins,
+                                                          const uint64_t* __restrict__ off,
+                                                          const uint32_t* __restrict__ src,
+                                                          const int32_t* __restrict__ w, uint32_t* __restrict__ cnt,
+                                                          const uint64_t* __restrict__ place, uint4* __restrict__ rec) {
+    extern __shared__ uint32_t bin[];   // counts, or the next place
+    // places of more than 32 bits are held relative to the bin's first
+    const bool wide = kWrite && place[static_cast<uint64_t>(bins) * gridDim.x] >> 32U != 0;
+    for (uint32_t b = threadIdx.x; b < bins; b += kOutThreads) {
+        const uint64_t at = static_cast<uint64_t>(b) * gridDim.x;
+        bin[b] = kWrite ? static_cast<uint32_t>(place[at + blockIdx.x] - (wide ? place[at] : 0)) : 0U;
+    }
+    __syncthreads();
+    const uint64_t first = blockIdx.x * per;
+    const uint64_t last = first + per < n ? first + per : n;
+    for (uint64_t t0 = first + (threadIdx.x & ~63U); t0 < last; t0 += kOutThreads) {
+        wave_pairs(t0, last, off, src, w, [&](uint64_t e, uint64_t t, uint32_t s, int32_t we) {
+            const uint32_t b = s >> shift;
+            const uint32_t at = atomicAdd(&bin[b], 1U);
+            if (kWrite) {
+                rec[at + (wide ? place[static_cast<uint64_t>(b) * gridDim.x] : 0)] =
+                    make_uint4(s, static_cast<uint32_t>(t), static_cast<uint32_t>(we), static_cast<uint32_t>(e));
+            }
+        });
+    }
+    if (!kWrite) {
+        __syncthreads();
+        for (uint32_t b = threadIdx.x; b < bins; b += kOutThreads) {
+            cnt[static_cast<uint64_t>(b) * gridDim.x + blockIdx.x] = bin[b];
+        }
+    }
+}
+
+// The counts of 2^shift sources become their exclusive prefix sums, the list offsets of sources
+// [s0, min(s0 + 2^shift, n)) at `base`.
+__device__ __forceinline__ void out_offsets(uint32_t* cnt, uint32_t shift, uint64_t s0, uint64_t n, uint64_t base,
+                                            uint64_t* __restrict__ out_off) {
+    constexpr uint32_t kMost = (1U << kOutMaxShift) / kOutThreads;
+    const uint32_t size = 1U << shift;
+    const uint32_t each = size > kOutThreads ? size / kOutThreads : 1U;
+    const uint32_t first = threadIdx.x * each;
+    const uint32_t lane = threadIdx.x & 63U;
+    const uint32_t wave = threadIdx.x >> 6U;
+    uint32_t v[kMost];
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kMost; k++) {
+        v[k] = k < each && first + k < size ? cnt[first + k] : 0U;
+        sum += v[k];
+    }
+    uint32_t inc = sum;
+#pragma unroll
+    for (uint32_t o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(inc, o);
+        inc += lane >= o ? y : 0U;
+    }
+    __syncthreads();   // every count is in registers: the array's start holds the waves' sums now
+    if (lane == 63) {
+        cnt[wave] = inc;
+    }
+    __syncthreads();
+    uint32_t run = inc - sum;
+#pragma unroll
+    for (uint32_t k = 0; k < kOutThreads / 64; k++) {
+        run += k < wave ? cnt[k] : 0U;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < kMost; k++) {
+        if (k < each && first + k < size) {
+            cnt[first + k] = run;
+            if (s0 + first + k < n) {
+                out_off[s0 + first + k] = base + run;
+            }
+            run += v[k];
+        }
+    }
+    __syncthreads();
+}
+
+// Block b sorts the records of bin b by source (order inside a source arbitrary).  Up to kOutStaged
+// records are read once, held in registers and written in order from LDS; a bin with more is read twice
+// and scattered.
+__global__ void __launch_bounds__(kOutThreads) k_out_sort(uint64_t n, uint32_t shift, uint32_t blocks,
+                                                          const uint64_t* __restrict__ place,
+                                                          const uint4* __restrict__ rec, uint64_t* __restrict__ out_off,
+                                                          uint2* __restrict__ out_pair, uint32_t* __restrict__ out_entry) {
+    extern __shared__ uint32_t cnt[];   // 2^shift counters, then the staging area
+    const uint32_t size = 1U << shift;
+    const uint64_t base = place[static_cast<uint64_t>(blockIdx.x) * blocks];
+    const uint64_t end = place[(static_cast<uint64_t>(blockIdx.x) + 1) * blocks];
+    const uint64_t s0 = static_cast<uint64_t>(blockIdx.x) << shift;
+    const uint32_t m = static_cast<uint32_t>(end - base);
+    for (uint32_t k = threadIdx.x; k < size; k += kOutThreads) {
+        cnt[k] = 0;
+    }
+    if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) {
+        out_off[n] = end;
+    }
+    __syncthreads();
+    if (m <= kOutStaged && shift <= kOutStageShift) {
+        uint2* pair = reinterpret_cast<uint2*>(cnt + size);
+        uint32_t* entry = reinterpret_cast<uint32_t*>(pair + kOutStaged);
+        uint4 r[kOutHeld];
+        uint32_t rank[kOutHeld];
+#pragma unroll
+        for (uint32_t k = 0; k < kOutHeld; k++) {
+            const uint32_t j = k * kOutThreads + threadIdx.x;
+            if (j < m) {
+                r[k] = rec[base + j];
+            }
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kOutHeld; k++) {
+            if (k * kOutThreads + threadIdx.x < m) {
+                rank[k] = atomicAdd(&cnt[r[k].x & (size - 1U)], 1U);
+            }
+        }
+        __syncthreads();
+        out_offsets(cnt, shift, s0, n, base, out_off);
+#pragma unroll
+        for (uint32_t k = 0; k < kOutHeld; k++) {
+            if (k * kOutThreads + threadIdx.x < m) {
+                const uint32_t at = cnt[r[k].x & (size - 1U)] + rank[k];
+                pair[at] = make_uint2(r[k].y, r[k].z);
+                entry[at] = r[k].w;
+            }
+        }
+        __syncthreads();
+        for (uint32_t j = threadIdx.x; j < m; j += kOutThreads) {
+            out_pair[base + j] = pair[j];
+            out_entry[base + j] = entry[j];
+        }
+        return;
+    }
+    for (uint32_t j = threadIdx.x; j < m; j += kOutThreads) {
+        atomicAdd(&cnt[rec[base + j].x & (size - 1U)], 1U);
+    }
+    __syncthreads();
+    out_offsets(cnt, shift, s0, n, base, out_off);
+    for (uint32_t j = threadIdx.x; j < m; j += kOutThreads) {
+        const uint4 r = rec[base + j];
+        const uint64_t at = base + atomicAdd(&cnt[r.x & (size - 1U)], 1U);
+        out_pair[at] = make_uint2(r.y, r.z);
+        out_entry[at] = r.w;
+    }
+}
+
+// The same in one block for at most kOutOneSources sources, from the graph itself.
+__global__ void __launch_bounds__(kOutThreads) k_out_one(uint64_t n, const uint64_t* __restrict__ off,
+                                                         const uint32_t* __restrict__ src,
+                                                         const int32_t* __restrict__ w, uint64_t* __restrict__ out_off,
+                                                         uint2* __restrict__ out_pair, uint32_t* __restrict__ out_entry) {
+    __shared__ uint32_t cnt[kOutOneSources];   // 2^11
+    __shared__ uint32_t total;
+    for (uint32_t k = threadIdx.x; k < kOutOneSources; k += kOutThreads) {
+        cnt[k] = 0;
+    }
+    if (threadIdx.x == 0) {
+        total = 0;
+    }
+    __syncthreads();
+    uint32_t mine = 0;
+    for (uint64_t t0 = threadIdx.x & ~63U; t0 < n; t0 += kOutThreads) {
+        wave_pairs(t0, n, off, src, w, [&](uint64_t, uint64_t, uint32_t s, int32_t) {
+            atomicAdd(&cnt[s], 1U);
+            mine++;
+        });
+    }
+    atomicAdd(&total, mine);
+    __syncthreads();
+    out_offsets(cnt, 11U, 0, n, 0, out_off);
+    for (uint64_t t0 = threadIdx.x & ~63U; t0 < n; t0 += kOutThreads) {
+        wave_pairs(t0, n, off, src, w, [&](uint64_t e, uint64_t t, uint32_t s, int32_t we) {
+            const uint32_t at = atomicAdd(&cnt[s], 1U);
+            out_pair[at] = make_uint2(static_cast<uint32_t>(t), static_cast<uint32_t>(we));
+            out_entry[at] = static_cast<uint32_t>(e);
+        });
+    }
+    if (threadIdx.x == 0) {
+        out_off[n] = total;
+    }
+}
+
 // ---------------------------------------------------------------- synaptic input by push
-
-// Non-zero pairs per source (out_cnt starts at zero).
-__global__ void k_out_count(uint64_t n, const uint64_t* __restrict__ off, const uint32_t* __restrict__ src,
-                            const int32_t* __restrict__ w, uint32_t* __restrict__ out_cnt) {
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    for (uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; t < n; t += stride) {
-        for (uint64_t e = off[t]; e < off[t + 1]; e++) {
-            if (w[e] != 0) {
-                atomicAdd(&out_cnt[src[e]], 1U);
-            }
-        }
-    }
-}
-
-// The pairs grouped by source at out_off (order inside a source arbitrary); out_cnt returns to zero.
-__global__ void k_out_scatter(uint64_t n, const uint64_t* __restrict__ off, const uint32_t* __restrict__ src,
-                              const int32_t* __restrict__ w, const uint64_t* __restrict__ out_off,
-                              uint32_t* __restrict__ out_cnt, uint32_t* __restrict__ out_tgt, int32_t* __restrict__ out_w) {
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    for (uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; t < n; t += stride) {
-        for (uint64_t e = off[t]; e < off[t + 1]; e++) {
-            const int32_t we = w[e];
-            if (we != 0) {
-                const uint32_t s = src[e];
-                const uint64_t pos = out_off[s] + atomicSub(&out_cnt[s], 1U) - 1U;
-                out_tgt[pos] = static_cast<uint32_t>(t);
-                out_w[pos] = we;
-            }
-        }
-    }
-}
 
 // acc[t] += the weights of the pairs whose source has fired set (acc starts at zero).
 __global__ void k_syn_push_all(uint64_t n, const uint8_t* __restrict__ fired, const uint64_t* __restrict__ out_off,
-                               const uint32_t* __restrict__ out_tgt, const int32_t* __restrict__ out_w,
-                               int32_t* __restrict__ acc) {
+                               const uint2* __restrict__ out_pair, int32_t* __restrict__ acc) {
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
     for (uint64_t s = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; s < n; s += stride) {
         if (fired[s] != 0) {
             for (uint64_t e = out_off[s]; e < out_off[s + 1]; e++) {
-                atomicAdd(&acc[out_tgt[e]], out_w[e]);
+                const uint2 tw = out_pair[e];
+                atomicAdd(&acc[tw.x], static_cast<int32_t>(tw.y));
             }
         }
     }
@@ -243,37 +472,6 @@ __device__ __forceinline__ bool unit_less(const Unit& a, const Unit& b) {
     return a.copy < b.copy;
 }
 
-// Lists of the out-entries of the sources that delete axons: counted, prefix-summed, scattered as
-// (entry, target).
-__global__ void k_del_out_count(uint64_t n, const uint64_t* __restrict__ off, const uint32_t* __restrict__ src,
-                                const int32_t* __restrict__ w, const uint32_t* __restrict__ deleted,
-                                uint32_t* __restrict__ ocnt) {
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    for (uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; t < n; t += stride) {
-        for (uint64_t e = off[t]; e < off[t + 1]; e++) {
-            const uint32_t s = src[e];
-            if (w[e] != 0 && deleted[s] != 0) {
-                atomicAdd(&ocnt[s], 1U);
-            }
-        }
-    }
-}
-
-__global__ void k_del_out_scatter(uint64_t n, const uint64_t* __restrict__ off, const uint32_t* __restrict__ src,
-                                  const int32_t* __restrict__ w, const uint32_t* __restrict__ deleted,
-                                  const uint64_t* __restrict__ ooff, uint32_t* __restrict__ ocnt,
-                                  uint2* __restrict__ olist) {
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    for (uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; t < n; t += stride) {
-        for (uint64_t e = off[t]; e < off[t + 1]; e++) {
-            const uint32_t s = src[e];
-            if (w[e] != 0 && deleted[s] != 0) {
-                olist[ooff[s] + atomicSub(&ocnt[s], 1U) - 1U] = make_uint2(static_cast<uint32_t>(e), static_cast<uint32_t>(t));
-            }
-        }
-    }
-}
-
 // The k-th smallest unit of a neuron (k >= 1), by k selection passes over its entries.  `entry(j)`
 // gives (partner, |weight|) of entry j < m, or |weight| 0 for entries that do not count.
 template <typename Entry>
@@ -306,7 +504,9 @@ __device__ __forceinline__ uint32_t local_id(const DelArgs& a, uint32_t i) {
 
 // Axons: source s deletes deleted[s] units among its outgoing pairs; each unit lowers the pair's
 // weight and disconnects one dendrite (of s's signal type) of the target.
-__global__ void k_del_axons(DelArgs a, const uint64_t* __restrict__ ooff, const uint2* __restrict__ olist) {
+// The lists by source hold the weights as they are before this kernel.
+__global__ void k_del_axons(DelArgs a, const uint64_t* __restrict__ out_off, const uint2* __restrict__ out_pair,
+                            const uint32_t* __restrict__ out_entry) {
     const uint32_t step = *a.step;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
     unsigned long long done = 0, short_of = 0;
@@ -315,15 +515,15 @@ __global__ void k_del_axons(DelArgs a, const uint64_t* __restrict__ ooff, const 
         if (want == 0) {
             continue;
         }
-        const uint64_t o = ooff[s];
-        const uint32_t m = static_cast<uint32_t>(ooff[s + 1] - o);
+        const uint64_t o = out_off[s];
+        const uint32_t m = static_cast<uint32_t>(out_off[s + 1] - o);
         const uint32_t g = a.net_of[s];
         const uint64_t seed = a.net_seed[g];
         const uint32_t self = local_id(a, static_cast<uint32_t>(s));
         auto entry = [&](uint32_t j) -> uint2 {
-            const uint2 et = olist[o + j];
-            const int32_t wt = a.w[et.x];
-            return make_uint2(local_id(a, et.y), static_cast<uint32_t>(wt < 0 ? -wt : wt));
+            const uint2 tw = out_pair[o + j];
+            const int32_t wt = static_cast<int32_t>(tw.y);
+            return make_uint2(local_id(a, tw.x), static_cast<uint32_t>(wt < 0 ? -wt : wt));
         };
         uint32_t units = 0;
         for (uint32_t j = 0; j < m; j++) {
@@ -337,7 +537,6 @@ __global__ void k_del_axons(DelArgs a, const uint64_t* __restrict__ ooff, const 
         const Unit last = kth_unit(seed, self, step, 0U, m, k, entry);
         const int sig = a.signal[s] != 0 ? 1 : 0;
         for (uint32_t j = 0; j < m; j++) {
-            const uint2 et = olist[o + j];
             const uint2 pw = entry(j);
             uint32_t sel = 0;
             for (uint32_t c = 0; c < pw.y; c++) {
@@ -345,9 +544,10 @@ __global__ void k_del_axons(DelArgs a, const uint64_t* __restrict__ ooff, const 
                 sel += unit_less(last, u) ? 0U : 1U;
             }
             if (sel != 0) {
-                a.w[et.x] -= unit_sign(a.w[et.x]) * static_cast<int32_t>(sel);
-                atomicSub(&a.conn[1 + sig][et.y], sel);
-                atomicAdd(&a.vac[1 + sig][et.y], sel);
+                const uint2 tw = out_pair[o + j];
+                a.w[out_entry[o + j]] -= unit_sign(static_cast<int32_t>(tw.y)) * static_cast<int32_t>(sel);
+                atomicSub(&a.conn[1 + sig][tw.x], sel);
+                atomicAdd(&a.vac[1 + sig][tw.x], sel);
                 done += sel;
             }
         }
@@ -408,17 +608,23 @@ __global__ void k_del_dendrites(DelArgs a, uint32_t type) {
     if (short_of != 0) atomicAdd(&a.counters[kCtrDelShort], short_of);
 }
 
+// The arrays of `cap` entries beside the graph's own.
+int net_alloc_scratch(rl_bh_ctx* c, uint64_t cap) {
+    NetGraph& g = c->net;
+    RL_TRY(dalloc(c, &g.scratch, cap));
+    g.src2 = reinterpret_cast<uint32_t*>(g.scratch);
+    g.w2 = reinterpret_cast<int32_t*>(g.src2 + cap);
+    RL_TRY(dalloc(c, &g.out_pair, cap));
+    RL_TRY(dalloc(c, &g.out_entry, cap));
+    g.cap = cap;
+    return RL_OK;
+}
+
 int net_alloc_edges(rl_bh_ctx* c, uint64_t cap) {
     NetGraph& g = c->net;
     RL_TRY(dalloc(c, &g.src, cap));
     RL_TRY(dalloc(c, &g.w, cap));
-    RL_TRY(dalloc(c, &g.src2, cap));
-    RL_TRY(dalloc(c, &g.w2, cap));
-    RL_TRY(dalloc(c, &g.olist, cap));
-    RL_TRY(dalloc(c, &g.out_tgt, cap));
-    RL_TRY(dalloc(c, &g.out_w, cap));
-    g.cap = cap;
-    return RL_OK;
+    return net_alloc_scratch(c, cap);
 }
 
 // Counts the accepted requests of the last commit per target into ncnt and their prefix into npre.
@@ -481,21 +687,21 @@ void net_free(rl_bh_ctx* c) {
     dfree(&g.src);
     dfree(&g.w);
     dfree(&g.off2);
-    dfree(&g.src2);
-    dfree(&g.w2);
     dfree(&g.ncnt);
     dfree(&g.npre);
-    dfree(&g.ocnt);
-    dfree(&g.ooff);
-    dfree(&g.olist);
     dfree(&g.out_off);
-    dfree(&g.out_cnt);
-    dfree(&g.out_tgt);
-    dfree(&g.out_w);
+    dfree(&g.out_pair);
+    dfree(&g.out_entry);
+    dfree(&g.bin_cnt);
+    dfree(&g.bin_off);
+    dfree(&g.scratch);
+    g.src2 = nullptr;
+    g.w2 = nullptr;
     dfree(&g.acc[0]);
     dfree(&g.acc[1]);
     g.cap = 0;
     g.ready = false;
+    g.out_valid = false;
     g.syn_valid = false;
 }
 
@@ -564,10 +770,9 @@ int net_init(rl_bh_ctx* c, uint64_t capacity, const uint64_t* in_offsets, const 
     RL_TRY(dalloc(c, &g.off2, n + 1));
     RL_TRY(dalloc(c, &g.ncnt, n));
     RL_TRY(dalloc(c, &g.npre, n + 1));
-    RL_TRY(dalloc(c, &g.ocnt, n));
-    RL_TRY(dalloc(c, &g.ooff, n + 1));
     RL_TRY(dalloc(c, &g.out_off, n + 1));
-    RL_TRY(dalloc(c, &g.out_cnt, n));
+    RL_TRY(dalloc(c, &g.bin_cnt, out_bins(n) * out_blocks(n)));
+    RL_TRY(dalloc(c, &g.bin_off, out_bins(n) * out_blocks(n) + 1));
     RL_TRY(dalloc(c, &g.acc[0], n));
     RL_TRY(dalloc(c, &g.acc[1], n));
     RL_TRY(net_alloc_edges(c, std::max<uint64_t>(capacity, 1)));
@@ -577,10 +782,10 @@ int net_init(rl_bh_ctx* c, uint64_t capacity, const uint64_t* in_offsets, const 
         RL_HIP(c, hipMemcpyAsync(g.src, src.data(), src.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s));
         RL_HIP(c, hipMemcpyAsync(g.w, w.data(), w.size() * sizeof(int32_t), hipMemcpyHostToDevice, s));
     }
-    RL_HIP(c, hipMemsetAsync(g.ocnt, 0, n * sizeof(uint32_t), s));
     RL_HIP(c, hipStreamSynchronize(s));
     g.entries_bound = src.size();
     g.ready = true;
+    g.out_valid = false;
     g.syn_valid = false;
     return RL_OK;
 }
@@ -617,26 +822,50 @@ int net_get(rl_bh_ctx* c, uint64_t capacity, uint64_t* in_offsets, uint32_t* sou
     return RL_OK;
 }
 
-// Rebuilds the out-edge lists from the graph and the accumulators from the fired status of
-// fired_buf[parity]: the state the step kernel expects at that parity.  Allocates nothing and reads
-// no count on the host, so a captured period can end with it.
-int enqueue_syn_sync(rl_bh_ctx* c, int parity) {
+// Groups the graph's non-zero pairs by source.  Allocates nothing and reads no count on the host, so a
+// captured period can end with it.
+int enqueue_out_lists(rl_bh_ctx* c) {
+    NetGraph& g = c->net;
+    const uint64_t n = c->n;
+    if (!g.ready || n == 0) {
+        return RL_OK;
+    }
+    hipStream_t s = c->stream;
+    if (n <= kOutOneSources && g.cap <= kOutOnePairs) {
+        k_out_one<<<1, kOutThreads, 0, s>>>(n, g.off, g.src, g.w, g.out_off, g.out_pair, g.out_entry);
+        RL_HIP(c, hipGetLastError());
+        return RL_OK;
+    }
+    const uint32_t shift = out_shift(n);
+    const uint32_t bins = static_cast<uint32_t>(out_bins(n));
+    const unsigned blocks = static_cast<unsigned>(out_blocks(n));
+    const uint64_t per = (n + blocks - 1) / blocks;
+    k_out_bins<false><<<blocks, kOutThreads, bins * sizeof(uint32_t), s>>>(n, per, shift, bins, g.off, g.src, g.w,
+                                                                           g.bin_cnt, nullptr, nullptr);
+    RL_HIP(c, hipGetLastError());
+    RL_TRY(scan_counts(c, g.bin_cnt, static_cast<uint64_t>(bins) * blocks, g.bin_off));
+    k_out_bins<true><<<blocks, kOutThreads, bins * sizeof(uint32_t), s>>>(n, per, shift, bins, g.off, g.src, g.w, nullptr,
+                                                                          g.bin_off, g.scratch);
+    RL_HIP(c, hipGetLastError());
+    const size_t lds = (sizeof(uint32_t) << shift) +
+                       (shift <= kOutStageShift ? kOutStaged * (sizeof(uint2) + sizeof(uint32_t)) : 0);
+    k_out_sort<<<bins, kOutThreads, lds, s>>>(n, shift, blocks, g.bin_off, g.scratch, g.out_off, g.out_pair, g.out_entry);
+    RL_HIP(c, hipGetLastError());
+    return RL_OK;
+}
+
+// The accumulators from the fired status of fired_buf[parity] and the lists by source: the state the step
+// kernel expects at that parity.  Capturable as well.
+int enqueue_syn_push(rl_bh_ctx* c, int parity) {
     NetGraph& g = c->net;
     const uint64_t n = c->n;
     if (!g.ready || n == 0 || !c->neurons.ready) {
         return RL_OK;
     }
-    hipStream_t s = c->stream;
-    RL_TRY(fill_u32(c, g.out_cnt, 0U, n, nullptr, 0));
-    k_out_count<<<kStreamBlocks, kBlock, 0, s>>>(n, g.off, g.src, g.w, g.out_cnt);
-    RL_HIP(c, hipGetLastError());
-    RL_TRY(scan_counts(c, g.out_cnt, n, g.out_off));
-    k_out_scatter<<<kStreamBlocks, kBlock, 0, s>>>(n, g.off, g.src, g.w, g.out_off, g.out_cnt, g.out_tgt, g.out_w);
-    RL_HIP(c, hipGetLastError());
     RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(g.acc[0]), 0U, n, nullptr, 0));
     RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(g.acc[1]), 0U, n, nullptr, 0));
-    k_syn_push_all<<<kStreamBlocks, kBlock, 0, s>>>(n, c->neurons.fired_buf[parity], g.out_off, g.out_tgt, g.out_w,
-                                                    g.acc[parity]);
+    k_syn_push_all<<<kStreamBlocks, kBlock, 0, c->stream>>>(n, c->neurons.fired_buf[parity], g.out_off, g.out_pair,
+                                                            g.acc[parity]);
     RL_HIP(c, hipGetLastError());
     return RL_OK;
 }
@@ -646,7 +875,11 @@ int syn_prepare(rl_bh_ctx* c) {
     if (!g.ready || g.syn_valid || c->n == 0 || !c->neurons.ready) {
         return RL_OK;
     }
-    RL_TRY(enqueue_syn_sync(c, c->neurons.parity));
+    if (!g.out_valid) {
+        RL_TRY(enqueue_out_lists(c));
+        g.out_valid = true;
+    }
+    RL_TRY(enqueue_syn_push(c, c->neurons.parity));
     g.syn_valid = true;
     return RL_OK;
 }
@@ -677,21 +910,14 @@ static int net_grow(rl_bh_ctx* c, uint64_t have, uint64_t need) {
     RL_HIP(c, hipStreamSynchronize(s));
     dfree(&g.src);
     dfree(&g.w);
-    dfree(&g.src2);
-    dfree(&g.w2);
-    dfree(&g.olist);
-    dfree(&g.out_tgt);
-    dfree(&g.out_w);
+    dfree(&g.scratch);
+    dfree(&g.out_pair);
+    dfree(&g.out_entry);
     g.src = src;
     g.w = w;
+    g.out_valid = false;
     g.syn_valid = false;
-    RL_TRY(dalloc(c, &g.src2, cap));
-    RL_TRY(dalloc(c, &g.w2, cap));
-    RL_TRY(dalloc(c, &g.olist, cap));
-    RL_TRY(dalloc(c, &g.out_tgt, cap));
-    RL_TRY(dalloc(c, &g.out_w, cap));
-    g.cap = cap;
-    return RL_OK;
+    return net_alloc_scratch(c, cap);
 }
 
 // Merges the counted synapses (ncnt, npre of the last commit), growing the arrays first when they
@@ -715,6 +941,7 @@ int net_append(rl_bh_ctx* c) {
     if (!c->net.ready || c->n == 0) {
         return RL_OK;
     }
+    c->net.out_valid = false;
     c->net.syn_valid = false;
     RL_TRY(enqueue_net_count(c));
     return net_merge_grow(c);
@@ -726,6 +953,7 @@ int net_append_retry(rl_bh_ctx* c) {
     if (!c->net.ready || c->n == 0) {
         return RL_OK;
     }
+    c->net.out_valid = false;
     c->net.syn_valid = false;
     RL_TRY(net_merge_grow(c));
     unsigned long long over = 0;
@@ -747,13 +975,7 @@ int enqueue_net_delete(rl_bh_ctx* c, int type) {
     hipStream_t s = c->stream;
     const DelArgs a = del_args(c, type);
     if (type == 0) {
-        // out-entries of the sources that delete axons (ocnt is zero between phases)
-        k_del_out_count<<<grid_for(n), kBlock, 0, s>>>(n, g.off, g.src, g.w, a.deleted, g.ocnt);
-        RL_HIP(c, hipGetLastError());
-        RL_TRY(scan_counts(c, g.ocnt, n, g.ooff));
-        k_del_out_scatter<<<grid_for(n), kBlock, 0, s>>>(n, g.off, g.src, g.w, a.deleted, g.ooff, g.ocnt, g.olist);
-        RL_HIP(c, hipGetLastError());
-        k_del_axons<<<grid_for(n), kBlock, 0, s>>>(a, g.ooff, g.olist);
+        k_del_axons<<<grid_for(n), kBlock, 0, s>>>(a, g.out_off, g.out_pair, g.out_entry);
     } else {
         k_del_dendrites<<<grid_for(n), kBlock, 0, s>>>(a, static_cast<uint32_t>(type));
     }

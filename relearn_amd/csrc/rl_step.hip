@@ -80,8 +80,7 @@ struct StepArgs {
     int32_t* acc_cur;
     int32_t* acc_next;
     const uint64_t* out_off;
-    const uint32_t* out_tgt;
-    const int32_t* out_w;
+    const uint2* out_pair;       // target, weight
     double conductance;
     // 1 / h and -1 / tau_ca, divided once on the host (IEEE division is correctly rounded on both
     // sides, so the values are the ones the reference's loops use)
@@ -107,18 +106,15 @@ __device__ __forceinline__ const T& at(const T* base, uint32_t i) {
 // Pairs are read four at a time, so that their loads overlap.
 __device__ __forceinline__ void push_out_pairs(const StepArgs& a, uint64_t e0, uint64_t e1) {
     for (uint64_t e = e0; e < e1; e += 4) {
-        uint32_t t[4];
-        int32_t w[4];
+        uint2 tw[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const bool in = e + k < e1;
-            t[k] = in ? a.out_tgt[e + k] : 0U;
-            w[k] = in ? a.out_w[e + k] : 0;
+            tw[k] = e + k < e1 ? a.out_pair[e + k] : make_uint2(0U, 0U);
         }
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            if (w[k] != 0) {
-                atomicAdd(&a.acc_next[t[k]], w[k]);
+            if (tw[k].y != 0) {
+                atomicAdd(&a.acc_next[tw[k].x], static_cast<int32_t>(tw[k].y));
             }
         }
     }
@@ -464,8 +460,7 @@ StepArgs step_args(rl_bh_ctx* c) {
         a.acc_cur = c->net.acc[s.parity];
         a.acc_next = c->net.acc[s.parity ^ 1];
         a.out_off = c->net.out_off;
-        a.out_tgt = c->net.out_tgt;
-        a.out_w = c->net.out_w;
+        a.out_pair = c->net.out_pair;
         a.conductance = s.p.synapse_conductance;
     }
     return a;
@@ -595,6 +590,11 @@ int enqueue_elements_commit(rl_bh_ctx* c) {
         return RL_OK;
     }
     RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(c->counters + kCtrDeleted), 0U, 4, nullptr, 0));
+    // axons are deleted among the pairs by source; a captured period with synaptic input starts with valid
+    // lists (rl_bh_graph_launch) and its steps leave the pairs alone
+    if (c->capturing ? s.p.synaptic_input == 0 : !c->net.out_valid) {
+        RL_TRY(enqueue_out_lists(c));
+    }
     for (int t = 0; t < 3; t++) {
         k_elements_update<<<grid_for(n), kBlock, 0, c->stream>>>(n, t * n, (t + 1) * n, s.grown, s.delta, c->conn[0],
                                                                   c->conn[1], c->conn[2], c->vac[0], c->vac[1], c->vac[2],
@@ -609,10 +609,10 @@ int neurons_commit(rl_bh_ctx* c, uint32_t update, uint32_t* deleted) {
     if (c->neurons.ready && c->n > 0) {
         RL_TRY(set_steps(c, 0, update));
     }
-    if (c->net.ready) {
-        c->net.syn_valid = false;   // deletions change the pairs
-    }
-    RL_TRY(enqueue_elements_commit(c));
+    const int status = enqueue_elements_commit(c);
+    c->net.out_valid = false;   // deletions change the pairs
+    c->net.syn_valid = false;
+    RL_TRY(status);
     if (deleted != nullptr && c->n > 0) {
         RL_HIP(c, hipMemcpyAsync(deleted, c->neurons.deleted, 3 * c->n * sizeof(uint32_t), hipMemcpyDeviceToHost,
                                  c->stream));
