@@ -261,7 +261,8 @@ int rl_neurons_init(rl_bh_ctx* ctx, const rl_step_params* p, const double* x, co
 /* One simulation step of NeuronModel::update_electrical_activity + calcium + synaptic element
  * deltas (Simulation.cpp:443-453): Izhikevich (IzhikevichModelCPU.cpp:75-125), calcium
  * (CalciumCalculatorCPU.cpp:40-103), growth curve (SynapticElementsCPU.cpp:25-49).  input: n values
- * for input_mode 0, else NULL.  step addresses the counter-based input draws. */
+ * for input_mode 0, else NULL; page-locked input is read in stream order after the call has returned.
+ * step addresses the counter-based input draws. */
 int rl_neurons_step(rl_bh_ctx* ctx, uint32_t step, const double* input);
 
 /* ElementBaseBase::update (ElementBaseBase.h:420-487) for the three element types: applies the

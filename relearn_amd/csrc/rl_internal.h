@@ -314,6 +314,8 @@ hipError_t scan_counts_on(hipStream_t s, const uint32_t* in, uint64_t n, uint64_
 hipError_t fill_u32_on(hipStream_t s, uint32_t* p, uint32_t value, uint64_t n, const uint64_t* n_dev, uint64_t cap);
 int fill_u32(rl_bh_ctx* c, uint32_t* p, uint32_t value, uint64_t n, const uint64_t* n_dev, uint64_t cap);
 int set_steps(rl_bh_ctx* c, uint32_t neuron_step, uint32_t update);
+// The device's address of a page-locked host range, or null (pageable, device or managed memory).
+void* mapped_host(const void* p, size_t bytes);
 
 // search (rl_search.hip, rl_search_coop.hip)
 int ensure_slots(rl_bh_ctx* c, uint64_t want);

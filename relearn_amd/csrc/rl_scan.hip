@@ -266,6 +266,24 @@ int fill_u32(rl_bh_ctx* c, uint32_t* p, uint32_t value, uint64_t n, const uint64
     return RL_OK;
 }
 
+void* mapped_host(const void* p, size_t bytes) {
+    if (p == nullptr || bytes == 0) {
+        return nullptr;
+    }
+    const char* const end = static_cast<const char*>(p) + bytes - 1;
+    hipPointerAttribute_t first{}, last{};
+    if (hipPointerGetAttributes(&first, p) != hipSuccess || hipPointerGetAttributes(&last, end) != hipSuccess) {
+        (void)hipGetLastError();   // memory that HIP does not know
+        return nullptr;
+    }
+    if (first.type != hipMemoryTypeHost || last.type != hipMemoryTypeHost || first.devicePointer == nullptr ||
+        static_cast<char*>(last.devicePointer) - static_cast<char*>(first.devicePointer) !=
+            static_cast<ptrdiff_t>(bytes - 1)) {
+        return nullptr;
+    }
+    return first.devicePointer;
+}
+
 int set_steps(rl_bh_ctx* c, uint32_t neuron_step, uint32_t update) {
     k_set_u32<<<1, 64, 0, c->stream>>>(c->d_steps, neuron_step, update);
     RL_HIP(c, hipGetLastError());
