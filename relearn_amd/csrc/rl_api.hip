@@ -195,8 +195,11 @@ int rl_bh_create(const rl_bh_config* cfg, rl_bh_ctx** out) {
     c->cfg = *cfg;
     if (hipSetDevice(cfg->device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
-        hipEventCreate(&c->ev2) != hipSuccess || hipEventCreate(&c->ev3) != hipSuccess) {
-        set_global_error("rl_bh_create: stream/event creation failed");
+        hipEventCreate(&c->ev2) != hipSuccess || hipEventCreate(&c->ev3) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void**>(&c->h_report), kReportWords * sizeof(unsigned long long),
+                      hipHostMallocMapped) != hipSuccess ||
+        hipHostGetDevicePointer(reinterpret_cast<void**>(&c->d_report), c->h_report, 0) != hipSuccess) {
+        set_global_error("rl_bh_create: stream, event or page-locked memory creation failed");
         delete c;
         return RL_EHIP;
     }
@@ -213,6 +216,9 @@ int rl_bh_destroy(rl_bh_ctx* c) {
         (void)hipStreamSynchronize(c->stream);
     }
     free_all(c);
+    if (c->h_report != nullptr) {
+        (void)hipHostFree(c->h_report);
+    }
     if (c->ev0 != nullptr) {
         (void)hipEventDestroy(c->ev0);
     }
@@ -600,9 +606,9 @@ int rl_bh_prepare_update_connectivity(rl_bh_ctx* c, const uint32_t* vacant_axons
     }
     RL_TRY(set_device(c));
     const uint32_t* h[3] = { vacant_axons, vacant_exc, vacant_inh };
-    for (int t = 0; t < 3 && c->n > 0; t++) {
-        RL_HIP(c, hipMemcpyAsync(c->vac[t], h[t], c->n * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    }
+    const size_t bytes = c->n * sizeof(uint32_t);
+    const CopyItem items[3] = { { c->vac[0], h[0], bytes }, { c->vac[1], h[1], bytes }, { c->vac[2], h[2], bytes } };
+    RL_TRY(copy_arrays(c, items, 3, hipMemcpyHostToDevice));
     return rl_bh_prepare_resident(c);
 }
 
@@ -616,9 +622,9 @@ int rl_bh_prepare_update_connectivity_device(rl_bh_ctx* c, const uint32_t* d_va,
     }
     RL_TRY(set_device(c));
     const uint32_t* d[3] = { d_va, d_ve, d_vi };
-    for (int t = 0; t < 3 && c->n > 0; t++) {
-        RL_HIP(c, hipMemcpyAsync(c->vac[t], d[t], c->n * sizeof(uint32_t), hipMemcpyDeviceToDevice, c->stream));
-    }
+    const size_t bytes = c->n * sizeof(uint32_t);
+    const CopyItem items[3] = { { c->vac[0], d[0], bytes }, { c->vac[1], d[1], bytes }, { c->vac[2], d[2], bytes } };
+    RL_TRY(copy_arrays(c, items, 3, hipMemcpyDeviceToDevice));
     return rl_bh_prepare_resident(c);
 }
 
@@ -628,7 +634,12 @@ int rl_bh_prepare_resident(rl_bh_ctx* c) {
     }
     RL_TRY(set_device(c));
     RL_TRY(prepare_tree(c));
+    if (c->n > 0) {
+        // the slots of the search, and their sum for the size of its buffers
+        RL_TRY(scan_counts(c, c->vac[0], c->n, c->slot_off, reinterpret_cast<uint64_t*>(c->d_report + kReportVacant)));
+    }
     RL_HIP(c, hipStreamSynchronize(c->stream));
+    c->vacant = c->n > 0 ? c->h_report[kReportVacant] : 0;
     c->prepared = true;
     c->searched_valid = false;
     return RL_OK;
@@ -660,12 +671,18 @@ int rl_bh_get_requests(rl_bh_ctx* c, uint64_t capacity, uint32_t* target, uint32
     RL_TRY(set_device(c));
     const uint64_t m = c->nreq;
     hipStream_t s = c->stream;
-    if (m > 0) {
-        if (target) RL_HIP(c, hipMemcpyAsync(target, c->req_target, m * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        if (source) RL_HIP(c, hipMemcpyAsync(source, c->req_source, m * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        if (signal) RL_HIP(c, hipMemcpyAsync(signal, c->req_signal, m, hipMemcpyDeviceToHost, s));
-        if (axon_ordinal) RL_HIP(c, hipMemcpyAsync(axon_ordinal, c->req_j, m * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    }
+    CopyItem items[4];
+    int count = 0;
+    auto add = [&](void* dst, const void* src, size_t bytes) {
+        if (dst != nullptr) {
+            items[count++] = { dst, src, bytes };
+        }
+    };
+    add(target, c->req_target, m * sizeof(uint32_t));
+    add(source, c->req_source, m * sizeof(uint32_t));
+    add(signal, c->req_signal, m);
+    add(axon_ordinal, c->req_j, m * sizeof(uint32_t));
+    RL_TRY(copy_arrays(c, items, count, hipMemcpyDeviceToHost));
     RL_HIP(c, hipStreamSynchronize(s));
     return RL_OK;
 }
@@ -710,7 +727,7 @@ int rl_bh_commit(rl_bh_ctx* c, uint32_t step, const uint64_t* order, uint64_t* c
     }
     RL_TRY(commit(c, step, order, created));
     c->prepared = false;  // vacancies changed: the tree must be prepared again before the next search
-    if (c->nreq > 0) {
+    if (c->nreq > 0 && c->net.ready) {   // without a graph the commit has already waited for its kernels
         RL_TRY(net_append(c));
         RL_HIP(c, hipStreamSynchronize(c->stream));
     }
@@ -725,9 +742,8 @@ int rl_bh_get_commit_result(rl_bh_ctx* c, uint64_t capacity, uint8_t* ok) {
         return fail(c, RL_EINVAL, "get_commit_result: capacity too small");
     }
     RL_TRY(set_device(c));
-    if (c->nreq > 0) {
-        RL_HIP(c, hipMemcpyAsync(ok, c->req_ok, c->nreq, hipMemcpyDeviceToHost, c->stream));
-    }
+    const CopyItem item{ ok, c->req_ok, c->nreq };
+    RL_TRY(copy_arrays(c, &item, 1, hipMemcpyDeviceToHost));
     RL_HIP(c, hipStreamSynchronize(c->stream));
     return RL_OK;
 }
@@ -800,11 +816,14 @@ int rl_bh_get_vacancies(rl_bh_ctx* c, uint32_t* va, uint32_t* ve, uint32_t* vi) 
     }
     RL_TRY(set_device(c));
     uint32_t* h[3] = { va, ve, vi };
-    for (int t = 0; t < 3 && c->n > 0; t++) {
+    CopyItem items[3];
+    int count = 0;
+    for (int t = 0; t < 3; t++) {
         if (h[t] != nullptr) {
-            RL_HIP(c, hipMemcpyAsync(h[t], c->vac[t], c->n * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+            items[count++] = { h[t], c->vac[t], c->n * sizeof(uint32_t) };
         }
     }
+    RL_TRY(copy_arrays(c, items, count, hipMemcpyDeviceToHost));
     RL_HIP(c, hipStreamSynchronize(c->stream));
     return RL_OK;
 }
@@ -1153,13 +1172,7 @@ int rl_bh_graph_launch(rl_bh_ctx* c, uint32_t first_step, uint32_t update, rl_bh
     }
     RL_HIP(c, hipEventRecord(c->ev1, s));
     unsigned long long h[kCounters];
-    RL_TRY(read_counters(c, h));
-    if (c->graph_appends && c->n > 0) {
-        uint64_t entries = 0;   // the graph's entries now (the stream is idle after the counters)
-        RL_HIP(c, hipMemcpyAsync(&entries, c->net.off + c->n, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-        RL_HIP(c, hipStreamSynchronize(s));
-        c->net.entries_bound = entries;
-    }
+    RL_TRY(read_counters(c, h, c->graph_appends ? &c->net.entries_bound : nullptr));
     float ms = 0.0f;
     RL_HIP(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     *stats = rl_bh_step_stats{};

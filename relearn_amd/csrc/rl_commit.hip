@@ -165,8 +165,12 @@ __global__ void __launch_bounds__(kCountThreads) k_commit_groups(uint64_t groups
 
 // Step 4, axon side: a source's requests are contiguous (found[i] of them at req_off[i]).
 __global__ void k_commit_axons(uint64_t n, const uint32_t* __restrict__ found, const uint64_t* __restrict__ req_off,
-                               const uint8_t* __restrict__ ok, uint32_t* __restrict__ vax, uint32_t* __restrict__ cax) {
+                               const uint8_t* __restrict__ ok, uint32_t* __restrict__ vax, uint32_t* __restrict__ cax,
+                               const unsigned long long* __restrict__ created, unsigned long long* __restrict__ report) {
     const uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
+    if (report != nullptr && i == 0) {
+        *report = *created;
+    }
     if (i >= n) {
         return;
     }
@@ -228,7 +232,9 @@ int enqueue_commit(rl_bh_ctx* c, const uint64_t* h_order) {
     k_commit_groups<<<count_blocks(groups), kCountThreads, 0, s>>>(groups, c->c_goff, c->vac[1], c->vac[2], c->conn[1], c->conn[2],
                                                      c->counters + kCtrCreated);
     RL_HIP(c, hipGetLastError());
-    k_commit_axons<<<grid_for(n), kBlock, 0, s>>>(n, c->found, c->req_off, c->req_ok, c->vac[0], c->conn[0]);
+    k_commit_axons<<<grid_for(n), kBlock, 0, s>>>(n, c->found, c->req_off, c->req_ok, c->vac[0], c->conn[0],
+                                                    c->counters + kCtrCreated,
+                                                    c->capturing ? nullptr : c->d_report + kCtrCreated);
     RL_HIP(c, hipGetLastError());
     return RL_OK;
 }
@@ -249,11 +255,9 @@ int commit(rl_bh_ctx* c, uint32_t step, const uint64_t* h_order, uint64_t* creat
     RL_TRY(set_steps(c, 0, step));
     RL_TRY(enqueue_commit(c, h_order));
     c->committed = true;
-    unsigned long long hc = 0;
-    RL_HIP(c, hipMemcpyAsync(&hc, c->counters + kCtrCreated, sizeof(hc), hipMemcpyDeviceToHost, c->stream));
     RL_HIP(c, hipStreamSynchronize(c->stream));
     if (created != nullptr) {
-        *created = hc;
+        *created = c->h_report[kCtrCreated];
     }
     return RL_OK;
 }

@@ -46,6 +46,13 @@ enum : int {
     kCounters = 19
 };
 
+// Words of rl_bh_ctx::h_report after the counters.
+enum : int {
+    kReportVacant = kCounters,   // vacant axons of the prepared update
+    kReportEntries,              // entries of the network graph
+    kReportWords
+};
+
 struct Status {
     int code = RL_OK;
     std::string msg;
@@ -176,6 +183,7 @@ struct rl_bh_ctx {
     // search results (slot layout: vacant axons per neuron at the exclusive prefix sum).  One
     // capacity, slots_cap, sizes every per-slot and per-request buffer: a neuron's requests are a
     // prefix of its slots, so there are never more requests than slots.
+    uint64_t vacant = 0;            // vacant axons of the prepared update
     uint64_t slots = 0;
     uint64_t slots_cap = 0;
     uint64_t* slot_off = nullptr;   // n + 1
@@ -208,6 +216,10 @@ struct rl_bh_ctx {
     uint64_t* wide = nullptr;        // n + 1: offsets of the active sources
     uint64_t* req_off = nullptr;     // n + 1
     unsigned long long* counters = nullptr;  // rl::kCounters device counters of the current update
+    // page-locked: what kernels report to the host (rl::kCounters counters, then the rl::kReport words),
+    // read after a synchronisation; and the device's address of it
+    unsigned long long* h_report = nullptr;
+    unsigned long long* d_report = nullptr;
     uint32_t* d_steps = nullptr;     // [0] first neuron step of a captured period, [1] plasticity update
     uint64_t* scan_part = nullptr;   // tile sums of scan_counts
     uint64_t scan_part_cap = 0;
@@ -308,21 +320,31 @@ void destroy_graph(rl_bh_ctx* c);
 
 // scans and fills (rl_scan.hip)
 uint64_t scan_scratch_entries(uint64_t n);
-int scan_counts(rl_bh_ctx* c, const uint32_t* in, uint64_t n, uint64_t* out);  // out[0..n], out[n] = total
+// out[0..n], out[n] = total; the total to *total as well unless it is null
+int scan_counts(rl_bh_ctx* c, const uint32_t* in, uint64_t n, uint64_t* out, uint64_t* total = nullptr);
 // the same on a given stream with scan_scratch_entries(n) tile sums at part (16-byte aligned operands)
-hipError_t scan_counts_on(hipStream_t s, const uint32_t* in, uint64_t n, uint64_t* out, uint64_t* part);
+hipError_t scan_counts_on(hipStream_t s, const uint32_t* in, uint64_t n, uint64_t* out, uint64_t* part,
+                          uint64_t* total = nullptr);
 hipError_t fill_u32_on(hipStream_t s, uint32_t* p, uint32_t value, uint64_t n, const uint64_t* n_dev, uint64_t cap);
 int fill_u32(rl_bh_ctx* c, uint32_t* p, uint32_t value, uint64_t n, const uint64_t* n_dev, uint64_t cap);
 int set_steps(rl_bh_ctx* c, uint32_t neuron_step, uint32_t update);
 // The device's address of a page-locked host range, or null (pageable, device or managed memory).
 void* mapped_host(const void* p, size_t bytes);
+// Arrays of one API call, copied on the context's stream.
+struct CopyItem {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+constexpr int kMaxCopies = 16;
+int copy_arrays(rl_bh_ctx* c, const CopyItem* items, int count, hipMemcpyKind kind);
 
 // search (rl_search.hip, rl_search_coop.hip)
 int ensure_slots(rl_bh_ctx* c, uint64_t want);
-int search_capacity(rl_bh_ctx* c);
 int enqueue_search(rl_bh_ctx* c);
 int find_targets(rl_bh_ctx* c, uint32_t step);
-int read_counters(rl_bh_ctx* c, unsigned long long* h);
+// the counters, and the network graph's entries into *entries unless it is null
+int read_counters(rl_bh_ctx* c, unsigned long long* h, uint64_t* entries = nullptr);
 int candidate_lists(rl_bh_ctx* c, uint64_t num_sources, const uint32_t* sources, uint64_t cap, uint32_t* nodes,
                     double* probs, uint32_t* counts);
 struct SearchArgs;

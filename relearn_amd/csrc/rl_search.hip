@@ -550,7 +550,8 @@ __global__ void __launch_bounds__(kBlock) k_candidates(SearchArgs a, const uint3
 
 __global__ void k_collect(unsigned long long* __restrict__ counters, const unsigned long long* __restrict__ cursor,
                           const uint64_t* __restrict__ slots,
-                          const uint64_t* __restrict__ requests, const uint64_t* __restrict__ active) {
+                          const uint64_t* __restrict__ requests, const uint64_t* __restrict__ active,
+                          unsigned long long* __restrict__ report) {
     if (threadIdx.x == 0) {
         counters[kCtrSlots] = *slots;
         counters[kCtrRequests] = *requests;
@@ -560,6 +561,21 @@ __global__ void k_collect(unsigned long long* __restrict__ counters, const unsig
             exec += cursor[x * kCursorStride + 1];
         }
         counters[kCtrTestsExec] += exec;
+    }
+    __syncthreads();
+    if (report != nullptr && threadIdx.x < kCounters) {
+        report[threadIdx.x] = counters[threadIdx.x];
+    }
+}
+
+// The counters, and the entries of the network graph, to the host's report.
+__global__ void k_report(const unsigned long long* __restrict__ counters, const uint64_t* __restrict__ entries,
+                         unsigned long long* __restrict__ report) {
+    if (threadIdx.x < kCounters) {
+        report[threadIdx.x] = counters[threadIdx.x];
+    }
+    if (entries != nullptr && threadIdx.x == 0) {
+        report[kReportEntries] = *entries;
     }
 }
 
@@ -656,15 +672,6 @@ SearchArgs search_args(rl_bh_ctx* c) {
     return a;
 }
 
-// Sizes the slot buffers for the resident vacancies (one host read of their sum).
-int search_capacity(rl_bh_ctx* c) {
-    RL_TRY(scan_counts(c, c->vac[0], c->n, c->slot_off));
-    uint64_t total = 0;
-    RL_HIP(c, hipMemcpyAsync(&total, c->slot_off + c->n, sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
-    RL_HIP(c, hipStreamSynchronize(c->stream));
-    return ensure_slots(c, total);
-}
-
 // The search of one update on the context's stream, driven by counts in device memory: slot
 // offsets, the active sources in Morton order, the search kernels, the dense requests.  No host
 // synchronisation, allocation or memset, so it can be captured into a graph.  The update index is
@@ -675,7 +682,9 @@ int enqueue_search(rl_bh_ctx* c) {
     if (n == 0) {
         return RL_OK;
     }
-    RL_TRY(scan_counts(c, c->vac[0], n, c->slot_off));
+    if (c->capturing) {   // the eager calls have prefix-summed the slots for the size of the buffers
+        RL_TRY(scan_counts(c, c->vac[0], n, c->slot_off));
+    }
     k_search_reset<<<kStreamBlocks, kBlock, 0, s>>>(n, c->slot_off + n, c->slots_cap, c->found, c->searched,
                                                     c->slot_target, c->slot_tests, c->counters, c->coop_cursor);
     RL_HIP(c, hipGetLastError());
@@ -733,16 +742,28 @@ int enqueue_search(rl_bh_ctx* c) {
     k_emit_requests<<<grid_for(n), kBlock, 0, s>>>(n, c->found, c->req_off, c->slot_off, c->slot_target, c->signal,
                                                     c->req_target, c->req_source, c->req_signal, c->req_j);
     RL_HIP(c, hipGetLastError());
-    k_collect<<<1, 64, 0, s>>>(c->counters, c->coop_cursor, c->slot_off + n, c->req_off + n, n_active);
+    k_collect<<<1, 64, 0, s>>>(c->counters, c->coop_cursor, c->slot_off + n, c->req_off + n, n_active,
+                               c->capturing ? nullptr : c->d_report);
     RL_HIP(c, hipGetLastError());
     return RL_OK;
 }
 
-int read_counters(rl_bh_ctx* c, unsigned long long* h) {
-    RL_HIP(c, hipMemcpyAsync(h, c->counters, kCounters * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream));
+// The counters as a kernel reported them, once the stream has run.
+static int take_report(rl_bh_ctx* c, unsigned long long* h) {
     RL_HIP(c, hipStreamSynchronize(c->stream));
+    std::copy(c->h_report, c->h_report + kCounters, h);
     if (h[kCtrSticky] != 0) {
         RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(c->counters + kCtrSticky), 0U, 2, nullptr, 0));
+    }
+    return RL_OK;
+}
+
+int read_counters(rl_bh_ctx* c, unsigned long long* h, uint64_t* entries) {
+    k_report<<<1, 64, 0, c->stream>>>(c->counters, entries != nullptr ? c->net.off + c->n : nullptr, c->d_report);
+    RL_HIP(c, hipGetLastError());
+    RL_TRY(take_report(c, h));
+    if (entries != nullptr) {
+        *entries = c->h_report[kReportEntries];
     }
     return RL_OK;
 }
@@ -761,13 +782,13 @@ int find_targets(rl_bh_ctx* c, uint32_t step) {
         c->searched_valid = true;
         return RL_OK;
     }
-    RL_TRY(search_capacity(c));
+    RL_TRY(ensure_slots(c, c->vacant));
     RL_TRY(set_steps(c, 0, step));
     RL_HIP(c, hipEventRecord(c->ev0, s));
     RL_TRY(enqueue_search(c));
     RL_HIP(c, hipEventRecord(c->ev1, s));
     unsigned long long h[kCounters];
-    RL_TRY(read_counters(c, h));
+    RL_TRY(take_report(c, h));   // from k_collect
     if (h[kCtrOverCap] != 0) {
         return fail(c, RL_ELIMIT, "vacant axons exceed the slot buffers");
     }

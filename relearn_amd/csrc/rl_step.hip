@@ -647,19 +647,24 @@ int neurons_get(rl_bh_ctx* c, double* x, double* u, double* ca, uint8_t* fired, 
         return fail(c, RL_ESTATE, "rl_neurons_get called before rl_neurons_init");
     }
     const uint64_t n = c->n;
-    hipStream_t st = c->stream;
-    if (x) RL_HIP(c, hipMemcpyAsync(x, s.x, n * sizeof(double), hipMemcpyDeviceToHost, st));
-    if (u) RL_HIP(c, hipMemcpyAsync(u, s.u, n * sizeof(double), hipMemcpyDeviceToHost, st));
-    if (ca) RL_HIP(c, hipMemcpyAsync(ca, s.ca, n * sizeof(double), hipMemcpyDeviceToHost, st));
-    if (fired) RL_HIP(c, hipMemcpyAsync(fired, s.fired, n, hipMemcpyDeviceToHost, st));
-    if (delta) RL_HIP(c, hipMemcpyAsync(delta, s.delta, 3 * n * sizeof(double), hipMemcpyDeviceToHost, st));
-    if (grown) RL_HIP(c, hipMemcpyAsync(grown, s.grown, 3 * n * sizeof(double), hipMemcpyDeviceToHost, st));
-    if (connected) {
-        for (int t = 0; t < 3; t++) {
-            RL_HIP(c, hipMemcpyAsync(connected + t * n, c->conn[t], n * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    CopyItem items[kMaxCopies];
+    int count = 0;
+    auto add = [&](void* dst, const void* src, size_t bytes) {
+        if (dst != nullptr && bytes != 0) {
+            items[count++] = { dst, src, bytes };
         }
+    };
+    add(x, s.x, n * sizeof(double));
+    add(u, s.u, n * sizeof(double));
+    add(ca, s.ca, n * sizeof(double));
+    add(fired, s.fired, n);
+    add(delta, s.delta, 3 * n * sizeof(double));
+    add(grown, s.grown, 3 * n * sizeof(double));
+    for (int t = 0; t < 3 && connected != nullptr; t++) {
+        add(connected + t * n, c->conn[t], n * sizeof(uint32_t));
     }
-    RL_HIP(c, hipStreamSynchronize(st));
+    RL_TRY(copy_arrays(c, items, count, hipMemcpyDeviceToHost));
+    RL_HIP(c, hipStreamSynchronize(c->stream));
     return RL_OK;
 }
 
