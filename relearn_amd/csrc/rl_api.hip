@@ -1100,8 +1100,8 @@ int rl_bh_graph_create(rl_bh_ctx* c, uint32_t steps, uint64_t max_vacant_axons) 
         if (status == RL_OK) status = enqueue_elements_commit(c);
     }
     if (status == RL_OK) status = prepare_tree(c);
-    if (status == RL_OK) status = enqueue_search(c);
-    if (status == RL_OK) status = enqueue_commit(c, nullptr);
+    if (status == RL_OK) status = enqueue_search(c, 0);
+    if (status == RL_OK) status = enqueue_commit(c, 0, nullptr);
     if (status == RL_OK) status = enqueue_net_append(c);
     // the next period's steps push over the pairs as this period left them
     if (status == RL_OK && c->neurons.ready && c->neurons.p.synaptic_input != 0) {

@@ -40,20 +40,25 @@ __global__ void k_rank_from_order(uint64_t m, const uint64_t* __restrict__ order
     }
 }
 
+constexpr uint32_t kUngrouped = 0xFFFFFFFFU;
+
 // Step 1.  The counter-based priority of request i is addressed like the draws: the network's seed,
-// the source's id inside its network, the update index and the axon ordinal.
+// the source's id inside its network, the update index (*step, or eager_step where step is null) and the
+// axon ordinal.  sidx starts as kUngrouped.
 __global__ void k_commit_count(uint64_t n, const uint64_t* __restrict__ n_req, const uint32_t* __restrict__ tgt,
                                const uint32_t* __restrict__ src, const uint8_t* __restrict__ sig,
                                const uint32_t* __restrict__ rj, const uint32_t* __restrict__ net_of,
                                const uint64_t* __restrict__ net_off, const uint64_t* __restrict__ net_seed,
-                               const uint32_t* __restrict__ step, int counter_order, uint64_t* __restrict__ prio,
-                               uint32_t* __restrict__ gcnt, uint32_t* __restrict__ pos, uint8_t* __restrict__ ok) {
+                               const uint32_t* __restrict__ step, uint32_t eager_step, int counter_order,
+                               uint64_t* __restrict__ prio, uint32_t* __restrict__ gcnt, uint32_t* __restrict__ pos,
+                               uint32_t* __restrict__ sidx, uint8_t* __restrict__ ok) {
     const uint64_t m = *n_req;
-    const uint32_t st = *step;
+    const uint32_t st = step != nullptr ? *step : eager_step;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
     for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < m; i += stride) {
         const uint32_t s = src[i];
         const uint32_t t = tgt[i];
+        sidx[i] = kUngrouped;
         if (counter_order) {
             const uint32_t g = net_of != nullptr ? net_of[s] : 0U;   // no table: one network
             prio[i] = commit_priority(net_seed[g], s - static_cast<uint32_t>(net_off[g]), st, rj[i]);
@@ -71,8 +76,6 @@ __global__ void k_commit_count(uint64_t n, const uint64_t* __restrict__ n_req, c
 // requests than vacancies is accepted here.  The others go to their group's offset plus the position
 // step 1 gave them (an arbitrary order inside the group: step 3 compares priorities, not positions).
 // Positions of accepted groups keep the sentinel kUngrouped.
-constexpr uint32_t kUngrouped = 0xFFFFFFFFU;
-
 __global__ void k_commit_scatter(uint64_t n, const uint64_t* __restrict__ n_req, const uint32_t* __restrict__ tgt,
                                  const uint32_t* __restrict__ src, const uint8_t* __restrict__ sig,
                                  const uint64_t* __restrict__ prio, const uint64_t* __restrict__ goff,
@@ -163,16 +166,21 @@ __global__ void __launch_bounds__(kCountThreads) k_commit_groups(uint64_t groups
     }
 }
 
-// Step 4, axon side: a source's requests are contiguous (found[i] of them at req_off[i]).
+// Step 4, axon side: a source's requests are contiguous (found[i] of them at req_off[i]).  Clears the network
+// graph's counts (unless ncnt is null) for the append that follows.
 __global__ void k_commit_axons(uint64_t n, const uint32_t* __restrict__ found, const uint64_t* __restrict__ req_off,
                                const uint8_t* __restrict__ ok, uint32_t* __restrict__ vax, uint32_t* __restrict__ cax,
-                               const unsigned long long* __restrict__ created, unsigned long long* __restrict__ report) {
+                               const unsigned long long* __restrict__ created, unsigned long long* __restrict__ report,
+                               uint32_t* __restrict__ ncnt) {
     const uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
     if (report != nullptr && i == 0) {
         *report = *created;
     }
     if (i >= n) {
         return;
+    }
+    if (ncnt != nullptr) {
+        ncnt[i] = 0;
     }
     const uint32_t f = found[i];
     if (f == 0) {
@@ -193,9 +201,9 @@ __global__ void k_commit_axons(uint64_t n, const uint32_t* __restrict__ found, c
 
 // The commit of the requests of the last search (count in req_off[n]) on the context's stream.  With
 // h_order (host, c->nreq entries, a permutation checked by the caller) the requests are processed in
-// that order; otherwise by counter-based priority with the update index d_steps[1].  h_order is the
-// only host input and is not allowed while capturing.
-int enqueue_commit(rl_bh_ctx* c, const uint64_t* h_order) {
+// that order; otherwise by counter-based priority with the update index d_steps[1] (captured) or eager_step.
+// h_order is not allowed while capturing.  The search has cleared the group counts and kCtrCreated.
+int enqueue_commit(rl_bh_ctx* c, uint32_t eager_step, const uint64_t* h_order) {
     const uint64_t n = c->n;
     hipStream_t s = c->stream;
     if (n == 0) {
@@ -205,8 +213,7 @@ int enqueue_commit(rl_bh_ctx* c, const uint64_t* h_order) {
         return fail(c, RL_ESTATE, "an explicit commit order cannot be captured");
     }
     const uint64_t groups = 2 * n;
-    RL_TRY(fill_u32(c, c->c_gcnt, 0U, groups, nullptr, 0));
-    RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(c->counters + kCtrCreated), 0U, 2, nullptr, 0));
+    const unsigned blocks = stream_blocks(c->slots_cap);   // a request per slot at most
     if (h_order != nullptr && c->nreq > 0) {
         const uint64_t m = c->nreq;
         RL_HIP(c, hipMemcpyAsync(c->c_order, h_order, m * sizeof(uint64_t), hipMemcpyHostToDevice, s));
@@ -216,17 +223,18 @@ int enqueue_commit(rl_bh_ctx* c, const uint64_t* h_order) {
     const uint64_t* n_req = c->req_off + n;
     // position of each request inside its group: the caller's order is no longer needed once ranked
     uint32_t* gpos = reinterpret_cast<uint32_t*>(c->c_order);
-    k_commit_count<<<kStreamBlocks, kBlock, 0, s>>>(n, n_req, c->req_target, c->req_source, c->req_signal, c->req_j,
-                                                    c->net_of, c->net_off, c->net_seed, c->d_steps + 1,
-                                                    h_order == nullptr ? 1 : 0, c->c_prio, c->c_gcnt, gpos, c->req_ok);
+    k_commit_count<<<blocks, kBlock, 0, s>>>(n, n_req, c->req_target, c->req_source, c->req_signal, c->req_j,
+                                                    c->net_of, c->net_off, c->net_seed,
+                                                    c->capturing ? c->d_steps + 1 : nullptr, eager_step,
+                                                    h_order == nullptr ? 1 : 0, c->c_prio, c->c_gcnt, gpos, c->c_sidx,
+                                                    c->req_ok);
     RL_HIP(c, hipGetLastError());
     RL_TRY(scan_counts(c, c->c_gcnt, groups, c->c_goff));
-    RL_TRY(fill_u32(c, c->c_sidx, kUngrouped, 0, c->c_goff + groups, c->slots_cap));
-    k_commit_scatter<<<kStreamBlocks, kBlock, 0, s>>>(n, n_req, c->req_target, c->req_source, c->req_signal, c->c_prio,
+    k_commit_scatter<<<blocks, kBlock, 0, s>>>(n, n_req, c->req_target, c->req_source, c->req_signal, c->c_prio,
                                                       c->c_goff, c->vac[1], c->vac[2], gpos, c->c_sprio, c->c_sidx,
                                                       c->req_ok);
     RL_HIP(c, hipGetLastError());
-    k_commit_rank<<<kStreamBlocks, kBlock, 0, s>>>(c->c_goff + groups, c->c_goff, c->c_sprio, c->c_sidx,
+    k_commit_rank<<<blocks, kBlock, 0, s>>>(c->c_goff + groups, c->c_goff, c->c_sprio, c->c_sidx,
                                                    c->req_target, c->req_signal, c->vac[1], c->vac[2], c->req_ok);
     RL_HIP(c, hipGetLastError());
     k_commit_groups<<<count_blocks(groups), kCountThreads, 0, s>>>(groups, c->c_goff, c->vac[1], c->vac[2], c->conn[1], c->conn[2],
@@ -234,7 +242,8 @@ int enqueue_commit(rl_bh_ctx* c, const uint64_t* h_order) {
     RL_HIP(c, hipGetLastError());
     k_commit_axons<<<grid_for(n), kBlock, 0, s>>>(n, c->found, c->req_off, c->req_ok, c->vac[0], c->conn[0],
                                                     c->counters + kCtrCreated,
-                                                    c->capturing ? nullptr : c->d_report + kCtrCreated);
+                                                    c->capturing ? nullptr : c->d_report + kCtrCreated,
+                                                    c->net.ready ? c->net.ncnt : nullptr);
     RL_HIP(c, hipGetLastError());
     return RL_OK;
 }
@@ -252,8 +261,7 @@ int commit(rl_bh_ctx* c, uint32_t step, const uint64_t* h_order, uint64_t* creat
     if (c->nreq == 0) {
         return RL_OK;
     }
-    RL_TRY(set_steps(c, 0, step));
-    RL_TRY(enqueue_commit(c, h_order));
+    RL_TRY(enqueue_commit(c, step, h_order));
     c->committed = true;
     RL_HIP(c, hipStreamSynchronize(c->stream));
     if (created != nullptr) {
@@ -307,8 +315,14 @@ static_assert(sizeof(NoallocHeader) <= 256, "header slot");
 
 __device__ __align__(256) unsigned char scratch[kNaBytes];
 
-__global__ void k_noalloc_setup(NoallocHeader* h, uint64_t m, uint64_t seed, uint32_t step) {
-    if (threadIdx.x == 0) {
+// The call's header, and the group counts cleared.
+__global__ void k_noalloc_setup(NoallocHeader* __restrict__ h, uint64_t m, uint64_t seed, uint32_t step,
+                                uint32_t* __restrict__ gcnt, uint64_t groups) {
+    const uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
+    if (i < groups) {
+        gcnt[i] = 0;
+    }
+    if (i == 0) {
         h->m = m;
         h->net_off = 0;
         h->seed = seed;
@@ -415,27 +429,26 @@ extern "C" int rl_bh_commit_requests_noalloc(uint64_t n, uint64_t m, const uint3
     auto* sidx = reinterpret_cast<uint32_t*>(base + kNaSidx);
     auto* gpos = reinterpret_cast<uint32_t*>(base + kNaPos);
     const uint64_t groups = 2 * n;
+    const unsigned blocks = stream_blocks(m);
     // the array keeps the last call's contents: everything read before it is written is set here
-    k_noalloc_setup<<<1, 64, 0, s>>>(hdr, m, network_seed, step);
+    k_noalloc_setup<<<grid_for(groups), kBlock, 0, s>>>(hdr, m, network_seed, step, gcnt, groups);
     RL_NA_HIP(hipGetLastError());
-    RL_NA_HIP(fill_u32_on(s, gcnt, 0U, groups, nullptr, 0));
-    k_commit_count<<<kStreamBlocks, kBlock, 0, s>>>(n, &hdr->m, d_target, d_source, d_signal, d_axon_ordinal, nullptr,
-                                                    &hdr->net_off, &hdr->seed, &hdr->step, 1, prio, gcnt, gpos, d_ok);
+    k_commit_count<<<blocks, kBlock, 0, s>>>(n, &hdr->m, d_target, d_source, d_signal, d_axon_ordinal, nullptr,
+                                                    &hdr->net_off, &hdr->seed, &hdr->step, 0, 1, prio, gcnt, gpos, sidx, d_ok);
     RL_NA_HIP(hipGetLastError());
     RL_NA_HIP(scan_counts_on(s, gcnt, groups, goff, part));
-    RL_NA_HIP(fill_u32_on(s, sidx, kUngrouped, 0, goff + groups, kNoallocMaxRequests));
-    k_commit_scatter<<<kStreamBlocks, kBlock, 0, s>>>(n, &hdr->m, d_target, d_source, d_signal, prio, goff,
+    k_commit_scatter<<<blocks, kBlock, 0, s>>>(n, &hdr->m, d_target, d_source, d_signal, prio, goff,
                                                       d_vacant_excitatory_dendrites, d_vacant_inhibitory_dendrites,
                                                       gpos, sprio, sidx, d_ok);
     RL_NA_HIP(hipGetLastError());
-    k_commit_rank<<<kStreamBlocks, kBlock, 0, s>>>(goff + groups, goff, sprio, sidx, d_target, d_signal,
+    k_commit_rank<<<blocks, kBlock, 0, s>>>(goff + groups, goff, sprio, sidx, d_target, d_signal,
                                                    d_vacant_excitatory_dendrites, d_vacant_inhibitory_dendrites, d_ok);
     RL_NA_HIP(hipGetLastError());
     k_commit_groups<<<count_blocks(groups), kCountThreads, 0, s>>>(groups, goff, d_vacant_excitatory_dendrites,
                                                      d_vacant_inhibitory_dendrites, d_connected_excitatory_dendrites,
                                                      d_connected_inhibitory_dendrites, &hdr->created);
     RL_NA_HIP(hipGetLastError());
-    k_commit_axons_by_request<<<kStreamBlocks, kBlock, 0, s>>>(&hdr->m, d_source, d_ok, d_vacant_axons,
+    k_commit_axons_by_request<<<blocks, kBlock, 0, s>>>(&hdr->m, d_source, d_ok, d_vacant_axons,
                                                                d_connected_axons);
     RL_NA_HIP(hipGetLastError());
     if (created != nullptr) {

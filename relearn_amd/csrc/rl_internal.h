@@ -17,6 +17,11 @@ constexpr uint32_t kLinkMask = (1U << kLinkBits) - 1U;
 constexpr uint32_t kNoTarget = 0xFFFFFFFFU;
 constexpr int kDrawsPerPass = 8;             // draws resolved per pick traversal
 constexpr unsigned kStreamBlocks = 2048;     // grid of the grid-stride kernels sized on the device
+// ... of which the host knows that they have at most `most` items: blocks of 256
+inline unsigned stream_blocks(uint64_t most, unsigned blocks = kStreamBlocks) {
+    const uint64_t b = (most + 255) / 256;
+    return b == 0 ? 1U : static_cast<unsigned>(b < blocks ? b : blocks);
+}
 constexpr int kCursorSlots = 8;              // work cursors of the persistent search waves, one per XCD
 constexpr int kCursorStride = 16;            // 64-bit words between cursors: a 128-byte line each (word 1: tests)
 constexpr uint32_t kMaxWavesPerCu = 24;      // slot tables are allocated for this many search waves per CU
@@ -108,7 +113,7 @@ struct NetGraph {
     uint64_t* bin_off = nullptr;
     uint4* scratch = nullptr;      // cap: the pairs in bins (source, target, weight, entry), or src2 and w2
     // per step parity the summed weights that the neurons which fired pushed to their targets for the next step
-    int32_t* acc[2] = { nullptr, nullptr };  // n each
+    int32_t* acc[2] = { nullptr, nullptr };  // n each, one allocation
     uint64_t cap = 0;
     // host: an upper bound of the graph's entries, exact after a call that synchronised with the device
     // and raised by each replay without stats by the most synapses a period can append
@@ -325,8 +330,7 @@ int scan_counts(rl_bh_ctx* c, const uint32_t* in, uint64_t n, uint64_t* out, uin
 // the same on a given stream with scan_scratch_entries(n) tile sums at part (16-byte aligned operands)
 hipError_t scan_counts_on(hipStream_t s, const uint32_t* in, uint64_t n, uint64_t* out, uint64_t* part,
                           uint64_t* total = nullptr);
-hipError_t fill_u32_on(hipStream_t s, uint32_t* p, uint32_t value, uint64_t n, const uint64_t* n_dev, uint64_t cap);
-int fill_u32(rl_bh_ctx* c, uint32_t* p, uint32_t value, uint64_t n, const uint64_t* n_dev, uint64_t cap);
+int fill_u32(rl_bh_ctx* c, uint32_t* p, uint32_t value, uint64_t n);
 int set_steps(rl_bh_ctx* c, uint32_t neuron_step, uint32_t update);
 // The device's address of a page-locked host range, or null (pageable, device or managed memory).
 void* mapped_host(const void* p, size_t bytes);
@@ -341,7 +345,7 @@ int copy_arrays(rl_bh_ctx* c, const CopyItem* items, int count, hipMemcpyKind ki
 
 // search (rl_search.hip, rl_search_coop.hip)
 int ensure_slots(rl_bh_ctx* c, uint64_t want);
-int enqueue_search(rl_bh_ctx* c);
+int enqueue_search(rl_bh_ctx* c, uint32_t eager_step);
 int find_targets(rl_bh_ctx* c, uint32_t step);
 // the counters, and the network graph's entries into *entries unless it is null
 int read_counters(rl_bh_ctx* c, unsigned long long* h, uint64_t* entries = nullptr);
@@ -372,10 +376,20 @@ inline uint64_t walk_min_default(const rl_bh_ctx* c) {
 inline uint64_t walk_min_sources(const rl_bh_ctx* c) {
     return (c->cfg.flags & RL_FLAG_WALK_ALWAYS) != 0 ? 0 : c->walk_min;
 }
+// An update can reach the walk's threshold only with as many neurons.  Below, the lists by type, the packed
+// records and the walk itself (five launches of 4-5 us) are left out; with eight more launches folded into
+// their neighbours, a 51,842-neuron update takes 826 us instead of 864, a 1,000-neuron FP64 update, which
+// never had the walk's, 233 instead of 271.
+inline bool may_walk(const rl_bh_ctx* c) {
+    return uses_walk(c) && c->n >= walk_min_sources(c);
+}
+// setting of the wave-per-source search for the updates of an FP32-mixed context below that threshold
+constexpr uint32_t kMixedWavesPerCu = 22;
+constexpr uint32_t kMixedChunk = 8;
 int launch_descend_lane(rl_bh_ctx* c, const SearchArgs& sa, const uint4* items, const unsigned long long* count);
 
 // commit (rl_commit.hip)
-int enqueue_commit(rl_bh_ctx* c, const uint64_t* h_order);
+int enqueue_commit(rl_bh_ctx* c, uint32_t eager_step, const uint64_t* h_order);
 int commit(rl_bh_ctx* c, uint32_t step, const uint64_t* h_order, uint64_t* created);
 
 // neuron step (rl_step.hip)

@@ -59,28 +59,25 @@ __global__ void k_net_count(const uint64_t* __restrict__ n_req, const uint8_t* _
     }
 }
 
-// The merge writes target t's list at off[t] + npre[t] of the second buffer, room for its old entries
-// and its new synapses; that layout must fit the capacity.
-__global__ void k_net_check(uint64_t n, const uint64_t* __restrict__ off, const uint64_t* __restrict__ npre,
-                            uint64_t cap, unsigned long long* __restrict__ counters) {
-    if (threadIdx.x == 0) {
-        const uint64_t add = npre[n];
-        const bool over = off[n] + add > cap;
+// New synapses staged per target at npre[t]: their sources (the weight follows from the source's
+// signal type).  ncnt returns to zero.  The merge writes target t's list at off[t] + npre[t] of the second
+// buffer, room for its old entries and its new synapses: an append that does not fit the capacity in
+// that layout is left out, and the counts stay.
+__global__ void k_net_stage(uint64_t n, const uint64_t* __restrict__ off, uint64_t cap,
+                            const uint64_t* __restrict__ n_req, const uint8_t* __restrict__ ok,
+                            const uint32_t* __restrict__ tgt, const uint32_t* __restrict__ rsrc,
+                            const uint64_t* __restrict__ npre, uint32_t* __restrict__ ncnt, uint32_t* __restrict__ stage,
+                            unsigned long long* __restrict__ counters) {
+    const uint64_t add = npre[n];
+    const bool over = off[n] + add > cap;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
         counters[kCtrNetOver] = over ? 1ULL : 0ULL;
         counters[kCtrNetNew] = over ? 0ULL : add;
         if (over) {
             counters[kCtrSticky] += 1ULL;
         }
     }
-}
-
-// New synapses staged per target at npre[t]: their sources (the weight follows from the source's
-// signal type).  ncnt returns to zero.
-__global__ void k_net_stage(const uint64_t* __restrict__ n_req, const uint8_t* __restrict__ ok,
-                            const uint32_t* __restrict__ tgt, const uint32_t* __restrict__ rsrc,
-                            const uint64_t* __restrict__ npre, uint32_t* __restrict__ ncnt, uint32_t* __restrict__ stage,
-                            const unsigned long long* __restrict__ counters) {
-    if (counters[kCtrNetOver] != 0) {
+    if (over) {
         return;
     }
     const uint64_t m = *n_req;
@@ -134,8 +131,9 @@ __global__ void k_net_merge(uint64_t n, const uint64_t* __restrict__ off, const 
     }
 }
 
-// Compacted lists back into the primary arrays, at the prefix sum noff of the merged counts.
-__global__ void k_net_copyback(uint64_t n, const uint64_t* __restrict__ off, const uint64_t* __restrict__ npre,
+// Compacted lists back into the primary arrays, at the prefix sum noff of the merged counts, which become
+// the offsets (a list's old offset is read by its own lane only).
+__global__ void k_net_copyback(uint64_t n, uint64_t* __restrict__ off, const uint64_t* __restrict__ npre,
                                const uint64_t* __restrict__ noff, const uint32_t* __restrict__ src2,
                                const int32_t* __restrict__ w2, uint32_t* __restrict__ src, int32_t* __restrict__ w,
                                const unsigned long long* __restrict__ counters) {
@@ -143,25 +141,15 @@ __global__ void k_net_copyback(uint64_t n, const uint64_t* __restrict__ off, con
         return;
     }
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    for (uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; t < n; t += stride) {
+    for (uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; t <= n; t += stride) {
         const uint64_t from = off[t] + npre[t];
         const uint64_t to = noff[t];
-        const uint64_t k = noff[t + 1] - to;
+        const uint64_t k = t < n ? noff[t + 1] - to : 0;
+        off[t] = to;
         for (uint64_t j = 0; j < k; j++) {
             src[to + j] = src2[from + j];
             w[to + j] = w2[from + j];
         }
-    }
-}
-
-__global__ void k_net_offsets(uint64_t n, const uint64_t* __restrict__ noff, uint64_t* __restrict__ off,
-                              const unsigned long long* __restrict__ counters) {
-    if (counters[kCtrNetOver] != 0) {
-        return;
-    }
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    for (uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; t <= n; t += stride) {
-        off[t] = noff[t];
     }
 }
 
@@ -627,12 +615,12 @@ int net_alloc_edges(rl_bh_ctx* c, uint64_t cap) {
     return net_alloc_scratch(c, cap);
 }
 
-// Counts the accepted requests of the last commit per target into ncnt and their prefix into npre.
+// Counts the accepted requests of the last commit per target into ncnt (cleared by the commit) and their
+// prefix into npre.
 int enqueue_net_count(rl_bh_ctx* c) {
     NetGraph& g = c->net;
     const uint64_t n = c->n;
-    RL_TRY(fill_u32(c, g.ncnt, 0U, n, nullptr, 0));
-    k_net_count<<<kStreamBlocks, kBlock, 0, c->stream>>>(c->req_off + n, c->req_ok, c->req_target, g.ncnt);
+    k_net_count<<<stream_blocks(c->slots_cap), kBlock, 0, c->stream>>>(c->req_off + n, c->req_ok, c->req_target, g.ncnt);
     RL_HIP(c, hipGetLastError());
     return scan_counts(c, g.ncnt, n, g.npre);
 }
@@ -643,18 +631,14 @@ int enqueue_net_merge(rl_bh_ctx* c) {
     NetGraph& g = c->net;
     const uint64_t n = c->n;
     hipStream_t s = c->stream;
-    k_net_check<<<1, 64, 0, s>>>(n, g.off, g.npre, g.cap, c->counters);
-    RL_HIP(c, hipGetLastError());
-    k_net_stage<<<kStreamBlocks, kBlock, 0, s>>>(c->req_off + n, c->req_ok, c->req_target, c->req_source, g.npre,
+    k_net_stage<<<stream_blocks(c->slots_cap), kBlock, 0, s>>>(n, g.off, g.cap, c->req_off + n, c->req_ok, c->req_target, c->req_source, g.npre,
                                                  g.ncnt, c->c_sidx, c->counters);
     RL_HIP(c, hipGetLastError());
     k_net_merge<<<grid_for(n), kBlock, 0, s>>>(n, g.off, g.npre, g.src, g.w, c->c_sidx, c->signal, g.src2, g.w2, g.ncnt,
                                                c->counters);
     RL_HIP(c, hipGetLastError());
     RL_TRY(scan_counts(c, g.ncnt, n, g.off2));
-    k_net_copyback<<<grid_for(n), kBlock, 0, s>>>(n, g.off, g.npre, g.off2, g.src2, g.w2, g.src, g.w, c->counters);
-    RL_HIP(c, hipGetLastError());
-    k_net_offsets<<<grid_for(n + 1), kBlock, 0, s>>>(n, g.off2, g.off, c->counters);
+    k_net_copyback<<<grid_for(n + 1), kBlock, 0, s>>>(n, g.off, g.npre, g.off2, g.src2, g.w2, g.src, g.w, c->counters);
     RL_HIP(c, hipGetLastError());
     return RL_OK;
 }
@@ -698,7 +682,7 @@ void net_free(rl_bh_ctx* c) {
     g.src2 = nullptr;
     g.w2 = nullptr;
     dfree(&g.acc[0]);
-    dfree(&g.acc[1]);
+    g.acc[1] = nullptr;
     g.cap = 0;
     g.ready = false;
     g.out_valid = false;
@@ -773,8 +757,8 @@ int net_init(rl_bh_ctx* c, uint64_t capacity, const uint64_t* in_offsets, const 
     RL_TRY(dalloc(c, &g.out_off, n + 1));
     RL_TRY(dalloc(c, &g.bin_cnt, out_bins(n) * out_blocks(n)));
     RL_TRY(dalloc(c, &g.bin_off, out_bins(n) * out_blocks(n) + 1));
-    RL_TRY(dalloc(c, &g.acc[0], n));
-    RL_TRY(dalloc(c, &g.acc[1], n));
+    RL_TRY(dalloc(c, &g.acc[0], 2 * n));
+    g.acc[1] = g.acc[0] + n;
     RL_TRY(net_alloc_edges(c, std::max<uint64_t>(capacity, 1)));
     hipStream_t s = c->stream;
     RL_HIP(c, hipMemcpyAsync(g.off, off.data(), (n + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, s));
@@ -862,9 +846,8 @@ int enqueue_syn_push(rl_bh_ctx* c, int parity) {
     if (!g.ready || n == 0 || !c->neurons.ready) {
         return RL_OK;
     }
-    RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(g.acc[0]), 0U, n, nullptr, 0));
-    RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(g.acc[1]), 0U, n, nullptr, 0));
-    k_syn_push_all<<<kStreamBlocks, kBlock, 0, c->stream>>>(n, c->neurons.fired_buf[parity], g.out_off, g.out_pair,
+    RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(g.acc[0]), 0U, 2 * n));   // both
+    k_syn_push_all<<<stream_blocks(n), kBlock, 0, c->stream>>>(n, c->neurons.fired_buf[parity], g.out_off, g.out_pair,
                                                             g.acc[parity]);
     RL_HIP(c, hipGetLastError());
     return RL_OK;

@@ -209,14 +209,9 @@ __global__ void __launch_bounds__(kScanBlock) k_scan_down(const uint32_t* __rest
     }
 }
 
-__global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t value, uint64_t n, const uint64_t* __restrict__ n_dev,
-                           uint64_t cap) {
-    uint64_t count = n;
-    if (n_dev != nullptr) {
-        count = *n_dev < cap ? *n_dev : cap;
-    }
+__global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t value, uint64_t n) {
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < count; i += stride) {
+    for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < n; i += stride) {
         p[i] = value;
     }
 }
@@ -321,13 +316,9 @@ int scan_counts(rl_bh_ctx* c, const uint32_t* in, uint64_t n, uint64_t* out, uin
     return RL_OK;
 }
 
-hipError_t fill_u32_on(hipStream_t s, uint32_t* p, uint32_t value, uint64_t n, const uint64_t* n_dev, uint64_t cap) {
-    k_fill_u32<<<kStreamBlocks, 256, 0, s>>>(p, value, n, n_dev, cap);
-    return hipGetLastError();
-}
-
-int fill_u32(rl_bh_ctx* c, uint32_t* p, uint32_t value, uint64_t n, const uint64_t* n_dev, uint64_t cap) {
-    RL_HIP(c, fill_u32_on(c->stream, p, value, n, n_dev, cap));
+int fill_u32(rl_bh_ctx* c, uint32_t* p, uint32_t value, uint64_t n) {
+    k_fill_u32<<<stream_blocks(n), 256, 0, c->stream>>>(p, value, n);
+    RL_HIP(c, hipGetLastError());
     return RL_OK;
 }
 

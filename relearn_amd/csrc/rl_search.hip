@@ -440,14 +440,35 @@ __global__ void __launch_bounds__(kBlock) k_descend_lane(SearchArgs a, const uin
     add_totals(a.counters, tot);
 }
 
+// End of a search: the dense requests in (source, axon ordinal) order, the commit's group counts cleared
+// for it, and (block 0) the update's counts, to the host's report as well unless it is null.
 __global__ void k_emit_requests(uint64_t n, const uint32_t* __restrict__ found, const uint64_t* __restrict__ req_off,
                                 const uint64_t* __restrict__ slot_off, const uint32_t* __restrict__ slot_target,
                                 const uint8_t* __restrict__ signal, uint32_t* __restrict__ rt, uint32_t* __restrict__ rs,
-                                uint8_t* __restrict__ rg, uint32_t* __restrict__ rj) {
+                                uint8_t* __restrict__ rg, uint32_t* __restrict__ rj, uint2* __restrict__ gcnt,
+                                const uint64_t* __restrict__ active, const unsigned long long* __restrict__ cursor,
+                                unsigned long long* __restrict__ counters, unsigned long long* __restrict__ report) {
+    if (blockIdx.x == 0) {
+        if (threadIdx.x == 0) {
+            counters[kCtrSlots] = slot_off[n];
+            counters[kCtrRequests] = req_off[n];
+            counters[kCtrActive] = *active;
+            unsigned long long exec = 0;
+            for (int x = 0; x < kCursorSlots; x++) {
+                exec += cursor[x * kCursorStride + 1];
+            }
+            counters[kCtrTestsExec] += exec;
+        }
+        __syncthreads();
+        if (report != nullptr && threadIdx.x < kCounters) {
+            report[threadIdx.x] = counters[threadIdx.x];
+        }
+    }
     const uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
     if (i >= n) {
         return;
     }
+    gcnt[i] = make_uint2(0U, 0U);
     const uint32_t f = found[i];
     const uint64_t o = req_off[i];
     const uint64_t s = slot_off[i];
@@ -459,13 +480,17 @@ __global__ void k_emit_requests(uint64_t n, const uint32_t* __restrict__ found, 
     }
 }
 
-// Start of a search: results and counters cleared, slots of this update initialised.  When the
-// update has more vacant axons than the slot buffers hold, kCtrOverCap is raised and no source is
-// searched (the update then changes nothing).
+// Start of a search: results and counters cleared, slots of this update initialised, the active sources
+// flagged in Morton order (unless flag is null), the update index of an eager call set (step_at not
+// null).  When the update has more vacant axons than the slot buffers hold, kCtrOverCap is raised and no
+// source is searched (the update then changes nothing).
 __global__ void k_search_reset(uint64_t n, const uint64_t* __restrict__ slot_total, uint64_t cap,
                                uint32_t* __restrict__ found, uint32_t* __restrict__ searched,
                                uint32_t* __restrict__ slot_target, uint32_t* __restrict__ slot_tests,
-                               unsigned long long* __restrict__ counters, unsigned long long* __restrict__ cursor) {
+                               unsigned long long* __restrict__ counters, unsigned long long* __restrict__ cursor,
+                               const uint32_t* __restrict__ order, const uint8_t* __restrict__ enabled,
+                               const uint32_t* __restrict__ vac, uint32_t* __restrict__ flag,
+                               uint32_t* __restrict__ step_at, uint32_t step) {
     const uint64_t total = *slot_total;
     const bool over = total > cap;
     const uint64_t slots = over ? 0 : total;
@@ -474,6 +499,10 @@ __global__ void k_search_reset(uint64_t n, const uint64_t* __restrict__ slot_tot
     for (uint64_t i = t0; i < n; i += stride) {
         found[i] = 0;
         searched[i] = 0;
+        if (flag != nullptr) {
+            const uint32_t src = order[i];
+            flag[i] = (!over && enabled[src] != 0 && vac[src] != 0) ? 1U : 0U;
+        }
     }
     for (uint64_t i = t0; i < slots; i += stride) {
         slot_target[i] = kNone;
@@ -492,15 +521,8 @@ __global__ void k_search_reset(uint64_t n, const uint64_t* __restrict__ slot_tot
         cursor[t0 * kCursorStride] = 0;
         cursor[t0 * kCursorStride + 1] = 0;
     }
-}
-
-__global__ void k_active_flags(uint64_t n, const uint32_t* __restrict__ order, const uint8_t* __restrict__ enabled,
-                               const uint32_t* __restrict__ vac, const unsigned long long* __restrict__ counters,
-                               uint32_t* __restrict__ flag) {
-    const uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
-    if (t < n) {
-        const uint32_t src = order[t];
-        flag[t] = (counters[kCtrOverCap] == 0 && enabled[src] != 0 && vac[src] != 0) ? 1U : 0U;
+    if (t0 == 0 && step_at != nullptr) {
+        *step_at = step;
     }
 }
 
@@ -548,26 +570,6 @@ __global__ void __launch_bounds__(kBlock) k_candidates(SearchArgs a, const uint3
     counts[t] = static_cast<uint32_t>(v.count);
 }
 
-__global__ void k_collect(unsigned long long* __restrict__ counters, const unsigned long long* __restrict__ cursor,
-                          const uint64_t* __restrict__ slots,
-                          const uint64_t* __restrict__ requests, const uint64_t* __restrict__ active,
-                          unsigned long long* __restrict__ report) {
-    if (threadIdx.x == 0) {
-        counters[kCtrSlots] = *slots;
-        counters[kCtrRequests] = *requests;
-        counters[kCtrActive] = *active;
-        unsigned long long exec = 0;
-        for (int x = 0; x < kCursorSlots; x++) {
-            exec += cursor[x * kCursorStride + 1];
-        }
-        counters[kCtrTestsExec] += exec;
-    }
-    __syncthreads();
-    if (report != nullptr && threadIdx.x < kCounters) {
-        report[threadIdx.x] = counters[threadIdx.x];
-    }
-}
-
 // The counters, and the entries of the network graph, to the host's report.
 __global__ void k_report(const unsigned long long* __restrict__ counters, const uint64_t* __restrict__ entries,
                          unsigned long long* __restrict__ report) {
@@ -584,10 +586,11 @@ __global__ void k_report(const unsigned long long* __restrict__ counters, const 
 int launch_descend_lane(rl_bh_ctx* c, const SearchArgs& sa, const uint4* items, const unsigned long long* count) {
     hipStream_t s = c->stream;
     const size_t lds = static_cast<size_t>(std::max<uint32_t>(c->tree.depth, 1U)) * kBlock * sizeof(uint32_t);
+    const unsigned blocks = stream_blocks(c->slots_cap, kStreamBlocks / 2);   // a descent per slot at most
     if (c->cfg.precision == RL_PREC_FP32_MIXED) {
-        k_descend_lane<true><<<kStreamBlocks / 2, kBlock, lds, s>>>(sa, items, count);
+        k_descend_lane<true><<<blocks, kBlock, lds, s>>>(sa, items, count);
     } else {
-        k_descend_lane<false><<<kStreamBlocks / 2, kBlock, lds, s>>>(sa, items, count);
+        k_descend_lane<false><<<blocks, kBlock, lds, s>>>(sa, items, count);
     }
     RL_HIP(c, hipGetLastError());
     return RL_OK;
@@ -675,8 +678,8 @@ SearchArgs search_args(rl_bh_ctx* c) {
 // The search of one update on the context's stream, driven by counts in device memory: slot
 // offsets, the active sources in Morton order, the search kernels, the dense requests.  No host
 // synchronisation, allocation or memset, so it can be captured into a graph.  The update index is
-// read from d_steps[1].
-int enqueue_search(rl_bh_ctx* c) {
+// read from d_steps[1], where an eager call's is set first.
+int enqueue_search(rl_bh_ctx* c, uint32_t eager_step) {
     const uint64_t n = c->n;
     hipStream_t s = c->stream;
     if (n == 0) {
@@ -685,20 +688,19 @@ int enqueue_search(rl_bh_ctx* c) {
     if (c->capturing) {   // the eager calls have prefix-summed the slots for the size of the buffers
         RL_TRY(scan_counts(c, c->vac[0], n, c->slot_off));
     }
-    k_search_reset<<<kStreamBlocks, kBlock, 0, s>>>(n, c->slot_off + n, c->slots_cap, c->found, c->searched,
-                                                    c->slot_target, c->slot_tests, c->counters, c->coop_cursor);
-    RL_HIP(c, hipGetLastError());
     const bool exact = (c->cfg.flags & RL_FLAG_EXACT_ORDER) != 0 || c->tree.depth == 0;
     // the group walk builds its own source lists (per dendrite type); the other kernels take the
     // active sources in Morton order
-    const bool walk = !exact && uses_walk(c);
+    const bool walk = !exact && may_walk(c);
+    k_search_reset<<<stream_blocks(std::max(n, c->slots_cap)), kBlock, 0, s>>>(n, c->slot_off + n, c->slots_cap, c->found, c->searched,
+                                                    c->slot_target, c->slot_tests, c->counters, c->coop_cursor, c->order,
+                                                    c->enabled, c->vac[0], walk ? nullptr : c->coop_flag,
+                                                    c->capturing ? nullptr : c->d_steps + 1, eager_step);
+    RL_HIP(c, hipGetLastError());
     const uint64_t* n_active = c->wide + n;
     if (walk) {
         n_active = c->walk_off + 2 * n;
     } else {
-        k_active_flags<<<grid_for(n), kBlock, 0, s>>>(n, c->order, c->enabled, c->vac[0], c->counters,
-                                                       c->coop_flag);
-        RL_HIP(c, hipGetLastError());
         RL_TRY(scan_counts(c, c->coop_flag, n, c->wide));
         k_scatter_active<<<grid_for(n), kBlock, 0, s>>>(n, c->coop_flag, c->wide, c->order, c->coop_work);
         RL_HIP(c, hipGetLastError());
@@ -732,18 +734,17 @@ int enqueue_search(rl_bh_ctx* c) {
         a.nwork = reinterpret_cast<const uint64_t*>(c->counters + kCtrOverflow);
     }
     if (mixed) {
-        k_search<true, true><<<kStreamBlocks / 8, kBlock, lds, s>>>(a);
+        k_search<true, true><<<stream_blocks(n, kStreamBlocks / 8), kBlock, lds, s>>>(a);
     } else {
-        k_search<false, true><<<kStreamBlocks / 8, kBlock, lds, s>>>(a);
+        k_search<false, true><<<stream_blocks(n, kStreamBlocks / 8), kBlock, lds, s>>>(a);
     }
     RL_HIP(c, hipGetLastError());
     // dense requests in (source, j) order
     RL_TRY(scan_counts(c, c->found, n, c->req_off));
     k_emit_requests<<<grid_for(n), kBlock, 0, s>>>(n, c->found, c->req_off, c->slot_off, c->slot_target, c->signal,
-                                                    c->req_target, c->req_source, c->req_signal, c->req_j);
-    RL_HIP(c, hipGetLastError());
-    k_collect<<<1, 64, 0, s>>>(c->counters, c->coop_cursor, c->slot_off + n, c->req_off + n, n_active,
-                               c->capturing ? nullptr : c->d_report);
+                                                    c->req_target, c->req_source, c->req_signal, c->req_j,
+                                                    reinterpret_cast<uint2*>(c->c_gcnt), n_active, c->coop_cursor,
+                                                    c->counters, c->capturing ? nullptr : c->d_report);
     RL_HIP(c, hipGetLastError());
     return RL_OK;
 }
@@ -753,7 +754,7 @@ static int take_report(rl_bh_ctx* c, unsigned long long* h) {
     RL_HIP(c, hipStreamSynchronize(c->stream));
     std::copy(c->h_report, c->h_report + kCounters, h);
     if (h[kCtrSticky] != 0) {
-        RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(c->counters + kCtrSticky), 0U, 2, nullptr, 0));
+        RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(c->counters + kCtrSticky), 0U, 2));
     }
     return RL_OK;
 }
@@ -783,12 +784,11 @@ int find_targets(rl_bh_ctx* c, uint32_t step) {
         return RL_OK;
     }
     RL_TRY(ensure_slots(c, c->vacant));
-    RL_TRY(set_steps(c, 0, step));
     RL_HIP(c, hipEventRecord(c->ev0, s));
-    RL_TRY(enqueue_search(c));
+    RL_TRY(enqueue_search(c, step));
     RL_HIP(c, hipEventRecord(c->ev1, s));
     unsigned long long h[kCounters];
-    RL_TRY(take_report(c, h));   // from k_collect
+    RL_TRY(take_report(c, h));   // from k_emit_requests
     if (h[kCtrOverCap] != 0) {
         return fail(c, RL_ELIMIT, "vacant axons exceed the slot buffers");
     }

@@ -796,7 +796,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kMix
         __syncthreads();
     }
     if (ln == 0 && acc_exec != 0) {
-        // beside the wave's XCD's cursor; k_collect adds the eight up
+        // beside the wave's XCD's cursor; k_emit_requests adds the eight up
         atomicAdd(&a.cursor[(blockIdx.x % kXcds) * kCursorStride + 1], acc_exec);
     }
 }
@@ -812,7 +812,7 @@ __global__ void __launch_bounds__(kCountThreads) k_finalize(SearchArgs s) {
     const bool over = s.counters[kCtrOverCap] != 0;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
     for (uint64_t src = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; src < s.n; src += stride) {
-        // the active sources of k_active_flags: enabled, with vacant axons, and no over-capacity update
+        // the active sources that k_search_reset flags: enabled, with vacant axons, and no over-capacity update
         if (over || s.enabled[src] == 0 || s.vac_axon[src] == 0 || s.found[src] == kOverflowMark) {
             continue;
         }
@@ -854,7 +854,11 @@ __global__ void __launch_bounds__(kCountThreads) k_finalize(SearchArgs s) {
 int launch_search_coop(rl_bh_ctx* c, const SearchArgs& sa) {
     const bool timed = !c->capturing;
     if (timed) RL_HIP(c, hipEventRecord(c->ev2, c->stream));
-    RL_TRY(launch_level1(c, sa, c->coop_work, sa.nwork, UINT64_MAX, c->coop_blocks, c->search_chunk));
+    if (uses_walk(c)) {   // the tuned setting is the walk's
+        RL_TRY(launch_level1(c, sa, c->coop_work, sa.nwork, UINT64_MAX, c->cus * kMixedWavesPerCu, kMixedChunk));
+    } else {
+        RL_TRY(launch_level1(c, sa, c->coop_work, sa.nwork, UINT64_MAX, c->coop_blocks, c->search_chunk));
+    }
     if (timed) RL_HIP(c, hipEventRecord(c->ev3, c->stream));
     RL_TRY(launch_descend_lane(c, sa, c->slow_items, c->counters + kCtrSlow));
     return launch_finalize(c, sa);

@@ -36,7 +36,8 @@
 // The walk pays off only when every wave has several groups (a group's walk is a chain of about 10^4
 // dependent steps): an update with fewer active sources than walk_min_sources() takes the
 // wave-per-source kernel, which is launched beside the walk; each returns at once unless the device's
-// active-source count is on its side.
+// active-source count is on its side.  A context with fewer neurons than that never walks, and its
+// updates launch the wave-per-source search alone.
 #include <algorithm>
 
 #include "rl_search_eval.h"
@@ -872,8 +873,8 @@ int launch_search_walk(rl_bh_ctx* c, const SearchArgs& sa) {
     if (timed) RL_HIP(c, hipEventRecord(c->ev2, s));
     if (a.run_from > 0) {
         // the wave-per-source kernel over the same lists (sources of each type in Morton order), at the
-        // setting its tuning picks for updates below the threshold (22 waves per CU, 8 sources per grab)
-        RL_TRY(launch_level1(c, sa, c->walk_list, n_active, a.run_from, c->cus * 22U, 8U));
+        // setting its tuning picks for updates below the threshold
+        RL_TRY(launch_level1(c, sa, c->walk_list, n_active, a.run_from, c->cus * kMixedWavesPerCu, kMixedChunk));
     }
     // the counting instantiation is a separate kernel: the counters change the register allocation of the walk
     const bool count = (c->cfg.flags & RL_FLAG_COUNT_WALK) != 0;

@@ -256,15 +256,21 @@ struct Retract {
     double r[3];
 };
 
-// Element types [k0 / n, k1 / n) of every neuron: index k = type * n + neuron.
+// Element types [k0 / n, k1 / n) of every neuron: index k = type * n + neuron.  The first lane clears the
+// deletion counters (unless counters is null).
 __global__ void k_elements_update(uint64_t n, uint64_t k0, uint64_t k1, double* __restrict__ grown,
                                   double* __restrict__ delta, uint32_t* __restrict__ c0, uint32_t* __restrict__ c1,
                                   uint32_t* __restrict__ c2, uint32_t* __restrict__ v0, uint32_t* __restrict__ v1,
-                                  uint32_t* __restrict__ v2, uint32_t* __restrict__ deleted, Retract rr) {
+                                  uint32_t* __restrict__ v2, uint32_t* __restrict__ deleted, Retract rr,
+                                  unsigned long long* __restrict__ counters) {
 #pragma clang fp contract(off)
     const uint64_t k = k0 + blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
     if (k >= k1) {
         return;
+    }
+    if (counters != nullptr && k == k0) {
+        counters[kCtrDeleted] = 0;
+        counters[kCtrDelShort] = 0;
     }
     const int t = static_cast<int>(k / n);
     const uint64_t i = k - static_cast<uint64_t>(t) * n;
@@ -593,11 +599,10 @@ int enqueue_elements_commit(rl_bh_ctx* c) {
     if (!c->net.ready) {
         k_elements_update<<<grid_for(3 * n), kBlock, 0, c->stream>>>(n, 0, 3 * n, s.grown, s.delta, c->conn[0], c->conn[1],
                                                                       c->conn[2], c->vac[0], c->vac[1], c->vac[2], s.deleted,
-                                                                      retract_of(s));
+                                                                      retract_of(s), nullptr);
         RL_HIP(c, hipGetLastError());
         return RL_OK;
     }
-    RL_TRY(fill_u32(c, reinterpret_cast<uint32_t*>(c->counters + kCtrDeleted), 0U, 4, nullptr, 0));
     // axons are deleted among the pairs by source; a captured period with synaptic input starts with valid
     // lists (rl_bh_graph_launch) and its steps leave the pairs alone
     if (c->capturing ? s.p.synaptic_input == 0 : !c->net.out_valid) {
@@ -606,7 +611,8 @@ int enqueue_elements_commit(rl_bh_ctx* c) {
     for (int t = 0; t < 3; t++) {
         k_elements_update<<<grid_for(n), kBlock, 0, c->stream>>>(n, t * n, (t + 1) * n, s.grown, s.delta, c->conn[0],
                                                                   c->conn[1], c->conn[2], c->vac[0], c->vac[1], c->vac[2],
-                                                                  s.deleted, retract_of(s));
+                                                                  s.deleted, retract_of(s),
+                                                                  t == 0 ? c->counters : nullptr);
         RL_HIP(c, hipGetLastError());
         RL_TRY(enqueue_net_delete(c, t));
     }
