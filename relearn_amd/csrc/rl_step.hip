@@ -103,20 +103,40 @@ __device__ __forceinline__ const T& at(const T* base, uint32_t i) {
 // A neuron that fired adds the weight of each of its out-pairs [e0, e1) to the target's input of the
 // next step (integer atomics: the sums do not depend on their order).  Few neurons fire per step, so
 // this replaces a gather over every in-edge of every neuron.
-// Pairs are read four at a time, so that their loads overlap.
+// The step reads the first kPushAhead pairs before the growth curves and the rest, kPushBatch at a time,
+// after them: a launch that fits the chip at once ends with the last wave that pushes, whose three
+// round trips (offsets, pairs, pairs) are then mostly behind the arithmetic.  Period of 100 steps with 8
+// pairs per neuron: 300,001 neurons 2,570 us with no pair ahead, 2,520 with 4, 2,450 with 8, 2,402 with 12 and
+// 2,410 with 16; 1,000 neurons 955, 929, 874, 828 and 834 us; 2M neurons 11.78, 11.69, 11.70, 11.74 and 11.96 ms.
+constexpr uint32_t kPushAhead = 12;
+constexpr uint32_t kPushBatch = 8;
+
+template <uint32_t kCount>
+__device__ __forceinline__ void load_pairs(const StepArgs& a, uint64_t e, uint64_t e1, uint2 (&tw)[kCount]) {
+#pragma unroll
+    for (uint32_t k = 0; k < kCount; k++) {
+        tw[k] = make_uint2(0U, 0U);
+        if (e + k < e1) {
+            tw[k] = a.out_pair[e + k];
+        }
+    }
+}
+
+template <uint32_t kCount>
+__device__ __forceinline__ void push_pairs(const StepArgs& a, const uint2 (&tw)[kCount]) {
+#pragma unroll
+    for (uint32_t k = 0; k < kCount; k++) {
+        if (tw[k].y != 0) {
+            atomicAdd(&a.acc_next[tw[k].x], static_cast<int32_t>(tw[k].y));
+        }
+    }
+}
+
 __device__ __forceinline__ void push_out_pairs(const StepArgs& a, uint64_t e0, uint64_t e1) {
-    for (uint64_t e = e0; e < e1; e += 4) {
-        uint2 tw[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            tw[k] = e + k < e1 ? a.out_pair[e + k] : make_uint2(0U, 0U);
-        }
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (tw[k].y != 0) {
-                atomicAdd(&a.acc_next[tw[k].x], static_cast<int32_t>(tw[k].y));
-            }
-        }
+    for (uint64_t e = e0; e < e1; e += kPushBatch) {
+        uint2 tw[kPushBatch];
+        load_pairs(a, e, e1, tw);
+        push_pairs(a, tw);
     }
 }
 
@@ -128,8 +148,9 @@ __device__ __forceinline__ void push_out_pairs(const StepArgs& a, uint64_t e0, u
 // divergent branches, vector keys for Philox and a loop over the substeps.  1M neurons without synaptic
 // input: 28.0 -> 25.5 us; 2M with it: 62 -> 57 us.  Fewer resident waves, so that rounds overlap, are
 // slower (6 blocks per CU instead of 8: +2%, 4: +6%).
-// kSub: substeps of a step (the reference's 10) unrolled, or 0 for p.h of any number.
-template <uint32_t kSub>
+// kSub: substeps of a step (the reference's 10) unrolled, or 0 for p.h of any number.  kSynaptic: with
+// synaptic input (its pairs in flight take 28 registers, which the step without it does not pay).
+template <uint32_t kSub, bool kSynaptic>
 __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
 #pragma clang fp contract(off)
     __shared__ double2 table[32];
@@ -150,8 +171,7 @@ __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
     double* const delta[3] = { a.delta, a.delta + a.n, a.delta + 2 * a.n };
     const double dl[3] = { at(delta[0], i), at(delta[1], i), at(delta[2], i) };
     double input = p.input_mode == 0 ? at(a.input, i) : 0.0;
-    const bool synaptic = a.acc_cur != nullptr;
-    const int32_t syn = synaptic ? at(a.acc_cur, i) : 0;
+    const int32_t syn = kSynaptic ? at(a.acc_cur, i) : 0;
     if (threadIdx.x < 32) {
         table[threadIdx.x] = make_double2(kExpTable[threadIdx.x][0], kExpTable[threadIdx.x][1]);
     }
@@ -161,7 +181,7 @@ __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
     }
     if (en == 0) {
         at(a.fired, i) = fprev;  // the step leaves a disabled neuron's status as it was
-        if (synaptic) {
+        if (kSynaptic) {
             at(a.acc_cur, i) = 0;
             if (fprev != 0) {
                 push_out_pairs(a, a.out_off[i], a.out_off[i + 1]);
@@ -186,7 +206,7 @@ __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
             }
         }
     }
-    if (synaptic) {
+    if (kSynaptic) {
         // SynapticEquallyWeightedActivityInputCPU::update_local_input: the weights of the in-edges
         // whose source fired in the previous step, times the conductance.  The sum was pushed by those
         // sources; it is an integer, which the reference's FP64 accumulation of integer weights
@@ -216,7 +236,7 @@ __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
     at(a.fired, i) = spiked ? 1 : 0;
     at(a.x, i) = xv;
     at(a.u, i) = uv;
-    const bool push = synaptic && spiked;
+    const bool push = kSynaptic && spiked;
     uint64_t e0 = 0, e1 = 0;   // read here, used at the end
     if (push) {
         e0 = a.out_off[i];
@@ -229,6 +249,10 @@ __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
         c += scale * (c * tau_inv + local_beta);
     }
     at(a.ca, i) = c;
+    uint2 tw[kPushAhead];
+    if (kSynaptic) {
+        load_pairs(a, e0, e1, tw);   // none unless the neuron fired
+    }
 #pragma unroll
     for (int t = 0; t < 3; t++) {
         const double eta = a.min_ca != nullptr ? at(a.min_ca + t * a.n, i) : p.eta[t];
@@ -238,15 +262,25 @@ __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
         at(delta[t], i) = dl[t] + dz * nu;
     }
     if (push) {
-        push_out_pairs(a, e0, e1);
+        push_pairs(a, tw);
+        push_out_pairs(a, e0 + kPushAhead, e1);
+    }
+}
+
+template <bool kSynaptic>
+void launch_step_of(const StepArgs& a, hipStream_t s) {
+    if (a.p.h == 10) {
+        k_step<10, kSynaptic><<<grid_for(a.n), kBlock, 0, s>>>(a);
+    } else {
+        k_step<0, kSynaptic><<<grid_for(a.n), kBlock, 0, s>>>(a);
     }
 }
 
 void launch_step(const StepArgs& a, hipStream_t s) {
-    if (a.p.h == 10) {
-        k_step<10><<<grid_for(a.n), kBlock, 0, s>>>(a);
+    if (a.acc_cur != nullptr) {
+        launch_step_of<true>(a, s);
     } else {
-        k_step<0><<<grid_for(a.n), kBlock, 0, s>>>(a);
+        launch_step_of<false>(a, s);
     }
 }
 
