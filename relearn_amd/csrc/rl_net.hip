@@ -46,6 +46,35 @@ __device__ __forceinline__ int32_t unit_sign(int32_t w) {
     return w < 0 ? -1 : 1;
 }
 
+// The lists of 64 neighbouring targets, whose entries [lo, lo + m) a wave goes through in order, so that
+// its loads are consecutive; a lane finds its entry's list by bisection over the 64 starts.
+struct WaveLists {
+    uint64_t lo;
+    uint32_t start;   // of this lane's list, relative to lo
+    uint32_t m;
+
+    // Entry j's list: the last one that starts at or before it.  For all lanes of the wave together.
+    __device__ __forceinline__ uint32_t list_of(uint32_t j) const {
+        uint32_t k = 0;
+#pragma unroll
+        for (uint32_t step = 32; step != 0; step >>= 1) {
+            const uint32_t at = __shfl(start, static_cast<int>(k + step));
+            k += at <= j ? step : 0U;
+        }
+        return k;
+    }
+};
+
+__device__ __forceinline__ WaveLists wave_lists(uint64_t t0, uint64_t t1, const uint64_t* __restrict__ off) {
+    const uint64_t t = t0 + (threadIdx.x & 63U);
+    const uint64_t mine = off[t < t1 ? t : t1];
+    WaveLists l;
+    l.lo = __shfl(static_cast<unsigned long long>(mine), 0);
+    l.start = static_cast<uint32_t>(mine - l.lo);
+    l.m = static_cast<uint32_t>(off[t0 + 64 < t1 ? t0 + 64 : t1] - l.lo);
+    return l;
+}
+
 // ---------------------------------------------------------------- append
 
 __global__ void k_net_count(const uint64_t* __restrict__ n_req, const uint8_t* __restrict__ ok,
@@ -91,28 +120,64 @@ __global__ void k_net_stage(uint64_t n, const uint64_t* __restrict__ off, uint64
     }
 }
 
-// One lane per target: its non-zero pairs, then its new synapses added to the pair of their source
-// or appended as a new pair.  ncnt[t] gets the merged count.
+// Target t's list, its non-zero pairs and then its new synapses (added to the pair of their source or
+// appended as a new pair), at off[t] + npre[t] of the second buffer; ncnt[t] gets its length.  A wave copies
+// the lists of 64 targets as they are; then the lanes whose target lost a pair or has new synapses, a
+// few in a hundred, close the gaps and add them.  One lane per list from end to end, whose loads were 32
+// bytes apart and followed one another, took 283 us for 16M pairs of 2M targets;
+// 102 us now (2.5 of about 5 TB/s).
 __global__ void k_net_merge(uint64_t n, const uint64_t* __restrict__ off, const uint64_t* __restrict__ npre,
                             const uint32_t* __restrict__ src, const int32_t* __restrict__ w,
                             const uint32_t* __restrict__ stage, const uint8_t* __restrict__ signal,
-                            uint32_t* __restrict__ src2, int32_t* __restrict__ w2, uint32_t* __restrict__ ncnt,
+                            uint32_t* src2, int32_t* w2, uint32_t* __restrict__ ncnt,
                             const unsigned long long* __restrict__ counters) {
     if (counters[kCtrNetOver] != 0) {
         return;
     }
+    const uint32_t lane = threadIdx.x & 63U;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    for (uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; t < n; t += stride) {
-        const uint64_t base = off[t] + npre[t];
-        uint32_t k = 0;
-        for (uint64_t e = off[t]; e < off[t + 1]; e++) {
-            if (w[e] != 0) {
-                src2[base + k] = src[e];
-                w2[base + k] = w[e];
-                k++;
+    for (uint64_t t0 = blockIdx.x * static_cast<uint64_t>(blockDim.x) + (threadIdx.x & ~63U); t0 < n; t0 += stride) {
+        const WaveLists l = wave_lists(t0, n, off);
+        const uint64_t t = t0 + lane < n ? t0 + lane : n;
+        const uint64_t before = npre[t];   // new synapses of the targets before
+        const uint64_t first = __shfl(static_cast<unsigned long long>(before), 0);
+        const uint32_t shift = static_cast<uint32_t>(before - first);
+        uint64_t gaps = 0;                 // lists with a pair of weight 0
+        for (uint32_t j0 = 0; j0 < l.m; j0 += 64) {
+            const uint32_t j = j0 + lane;
+            const bool in = j < l.m;
+            const uint32_t s = in ? src[l.lo + j] : 0U;
+            const int32_t we = in ? w[l.lo + j] : 1;
+            const uint32_t k = l.list_of(j);
+            const uint64_t to = l.lo + j + first + __shfl(shift, static_cast<int>(k));
+            if (in) {
+                src2[to] = s;
+                w2[to] = we;
+            }
+            for (uint64_t zero = __ballot(we == 0); zero != 0; zero &= zero - 1) {
+                gaps |= 1ULL << __shfl(k, __ffsll(static_cast<unsigned long long>(zero)) - 1);
             }
         }
-        for (uint64_t q = npre[t]; q < npre[t + 1]; q++) {
+        __threadfence_block();   // the wave's copies before its lanes' reads
+        if (t >= n) {
+            continue;
+        }
+        const uint64_t base = l.lo + l.start + before;
+        const uint64_t end = npre[t + 1];
+        uint32_t k = static_cast<uint32_t>(off[t + 1] - off[t]);
+        if ((gaps >> lane & 1ULL) != 0) {
+            const uint32_t had = k;
+            k = 0;
+            for (uint32_t j = 0; j < had; j++) {
+                const int32_t we = w2[base + j];
+                if (we != 0) {
+                    src2[base + k] = src2[base + j];
+                    w2[base + k] = we;
+                    k++;
+                }
+            }
+        }
+        for (uint64_t q = before; q < end; q++) {
             const uint32_t s = stage[q];
             const int32_t dw = signal[s] != 0 ? -1 : 1;
             uint32_t j = 0;
@@ -132,7 +197,8 @@ __global__ void k_net_merge(uint64_t n, const uint64_t* __restrict__ off, const 
 }
 
 // Compacted lists back into the primary arrays, at the prefix sum noff of the merged counts, which become
-// the offsets (a list's old offset is read by its own lane only).
+// the offsets (a list's old offset is read by its own lane only).  Copied by the wave as in k_net_merge:
+// 226 -> 64 us for 16M pairs of 2M targets (4 TB/s).
 __global__ void k_net_copyback(uint64_t n, uint64_t* __restrict__ off, const uint64_t* __restrict__ npre,
                                const uint64_t* __restrict__ noff, const uint32_t* __restrict__ src2,
                                const int32_t* __restrict__ w2, uint32_t* __restrict__ src, int32_t* __restrict__ w,
@@ -140,15 +206,29 @@ __global__ void k_net_copyback(uint64_t n, uint64_t* __restrict__ off, const uin
     if (counters[kCtrNetOver] != 0) {
         return;
     }
+    const uint32_t lane = threadIdx.x & 63U;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    for (uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; t <= n; t += stride) {
-        const uint64_t from = off[t] + npre[t];
-        const uint64_t to = noff[t];
-        const uint64_t k = t < n ? noff[t + 1] - to : 0;
-        off[t] = to;
-        for (uint64_t j = 0; j < k; j++) {
-            src[to + j] = src2[from + j];
-            w[to + j] = w2[from + j];
+    for (uint64_t t0 = blockIdx.x * static_cast<uint64_t>(blockDim.x) + (threadIdx.x & ~63U); t0 < n; t0 += stride) {
+        const WaveLists l = wave_lists(t0, n, noff);
+        const uint64_t t = t0 + lane;
+        // how far this lane's list moves; it moves at least as far as the list before it
+        uint64_t moves = 0;
+        if (t < n) {
+            moves = off[t] + npre[t] - (l.lo + l.start);
+            off[t] = l.lo + l.start;
+        }
+        if (t0 + 64 >= n && lane == 0) {
+            off[n] = l.lo + l.m;
+        }
+        const uint64_t first = __shfl(static_cast<unsigned long long>(moves), 0);
+        const uint32_t more = static_cast<uint32_t>(moves - first);
+        for (uint32_t j0 = 0; j0 < l.m; j0 += 64) {
+            const uint32_t j = j0 + lane;
+            const uint64_t from = l.lo + j + first + __shfl(more, static_cast<int>(l.list_of(j)));
+            if (j < l.m) {
+                src[l.lo + j] = src2[from];
+                w[l.lo + j] = w2[from];
+            }
         }
     }
 }
@@ -200,29 +280,19 @@ uint64_t out_blocks(uint64_t n) {
     return std::min<uint64_t>(kOutBlocks, (n + kOutThreads - 1) / kOutThreads);
 }
 
-// f(entry, target, source, weight) for the non-zero pairs of targets [t0, min(t0 + 64, t1)): the wave reads the
-// entries in order; a lane finds its entry's target by bisection over the 64 offsets.
+// f(entry, target, source, weight) for the non-zero pairs of targets [t0, min(t0 + 64, t1)).
 template <typename F>
 __device__ __forceinline__ void wave_pairs(uint64_t t0, uint64_t t1, const uint64_t* __restrict__ off,
                                            const uint32_t* __restrict__ src, const int32_t* __restrict__ w, F f) {
-    const uint32_t lane = threadIdx.x & 63U;
-    const uint64_t mine = off[t0 + lane < t1 ? t0 + lane : t1];
-    const uint64_t lo = __shfl(static_cast<unsigned long long>(mine), 0);
-    const uint32_t rel = static_cast<uint32_t>(mine - lo);
-    const uint32_t m = static_cast<uint32_t>(off[t0 + 64 < t1 ? t0 + 64 : t1] - lo);
-    for (uint32_t j0 = 0; j0 < m; j0 += 64) {
-        const uint32_t j = j0 + lane;
-        const bool in = j < m;
-        const uint32_t s = in ? src[lo + j] : 0U;
-        const int32_t we = in ? w[lo + j] : 0;
-        uint32_t k = 0;   // the last target whose list starts at or before j
-#pragma unroll
-        for (uint32_t step = 32; step != 0; step >>= 1) {
-            const uint32_t start = __shfl(rel, static_cast<int>(k + step));
-            k += start <= j ? step : 0U;
-        }
+    const WaveLists l = wave_lists(t0, t1, off);
+    for (uint32_t j0 = 0; j0 < l.m; j0 += 64) {
+        const uint32_t j = j0 + (threadIdx.x & 63U);
+        const bool in = j < l.m;
+        const uint32_t s = in ? src[l.lo + j] : 0U;
+        const int32_t we = in ? w[l.lo + j] : 0;
+        const uint32_t k = l.list_of(j);
         if (we != 0) {
-            f(lo + j, t0 + k, s, we);
+            f(l.lo + j, t0 + k, s, we);
         }
     }
 }
@@ -638,7 +708,7 @@ int enqueue_net_merge(rl_bh_ctx* c) {
                                                c->counters);
     RL_HIP(c, hipGetLastError());
     RL_TRY(scan_counts(c, g.ncnt, n, g.off2));
-    k_net_copyback<<<grid_for(n + 1), kBlock, 0, s>>>(n, g.off, g.npre, g.off2, g.src2, g.w2, g.src, g.w, c->counters);
+    k_net_copyback<<<grid_for(n), kBlock, 0, s>>>(n, g.off, g.npre, g.off2, g.src2, g.w2, g.src, g.w, c->counters);
     RL_HIP(c, hipGetLastError());
     return RL_OK;
 }

@@ -1,5 +1,6 @@
 """The pairs grouped by source: what fired sources push and what axons are deleted among, at the sizes
-where the grouping changes (one block, bins of 256 to 1,024 sources), with uneven lists and pairs whose weight is 0."""
+where the grouping changes (one block, bins of 256 to 1,024 sources), with uneven lists and pairs whose weight is 0;
+and the append to lists that are empty, long or hold pairs whose weight is 0."""
 from __future__ import annotations
 
 import numpy as np
@@ -79,4 +80,46 @@ def test_pushes_and_axon_deletion(oracle, n, room):
     w = w2
     step(2)   # the lists hold the pairs that are left
     step(3)
+    g.close()
+
+
+@pytest.mark.parametrize("n,room", [(2, 40), (63, 400), (64, 400), (65, 0), (3001, 0), (3001, 20000)])
+def test_append_to_uneven_lists(n, room):
+    print("[gpu-case] append to uneven lists,", n, "neurons, room", room, flush=True)
+    rng = np.random.default_rng(n + room)
+    off, src, w = _graph(n, rng)
+    tgt = np.repeat(np.arange(n), np.diff(off.astype(np.int64)))
+    signal = (np.arange(n) % 5 == 0).astype(np.uint8)
+    conn = np.zeros((3, n), np.uint32)
+    np.add.at(conn[0], src, np.abs(w).astype(np.uint32))
+    np.add.at(conn[1], tgt[w > 0], w[w > 0].astype(np.uint32))
+    np.add.at(conn[2], tgt[w < 0], np.abs(w[w < 0]).astype(np.uint32))
+    p = StepParams.izhikevich(input_mode=0)
+    for k in range(3):
+        p.eta[k], p.nu[k] = 0.0, (3.0 if k == 0 else 0.0)   # axons shrink by about three elements
+    g = BarnesHutHIP((0, 0, 0), (1000, 1000, 1000), seed=4)
+    g.init(rng.random((n, 3)) * 1000.0, signal)
+    g.net_init(len(src) + room, off, src, w)
+    g.neurons_init(p, np.full(n, 0.1), ca=np.full(n, 0.9), grown=conn.astype(np.float64).ravel(), connected=conn.ravel())
+    gaps = 0
+    for update in range(3):
+        if update == 1:
+            g.neurons_step(0, np.full(n, 5.0))
+            g.neurons_commit_elements(update)
+        off, src, w = g.net_get_edges()
+        tgt = np.repeat(np.arange(n), np.diff(off.astype(np.int64)))
+        gaps += int((w == 0).sum())
+        expect = {k: v for k, v in zip(zip(tgt.tolist(), src.tolist()), w.tolist()) if v != 0}
+        g.prepare_update_connectivity(*[rng.poisson(m, n).astype(np.uint32) for m in (2.0, 1.5, 1.5)])
+        m = g.find_target_neurons(update)
+        g.commit(update)
+        req, ok = g.get_requests(m), np.asarray(g.get_commit_result(m))
+        new_tgt, new_src = np.asarray(req[0])[ok != 0], np.asarray(req[1])[ok != 0]
+        for t, s in zip(new_tgt.tolist(), new_src.tolist()):
+            expect[(t, s)] = expect.get((t, s), 0) + (-1 if signal[s] else 1)
+        off, src, w = g.net_get_edges()
+        tgt = np.repeat(np.arange(n), np.diff(off.astype(np.int64)))
+        assert len(src) == len(expect)
+        assert dict(zip(zip(tgt.tolist(), src.tolist()), w.tolist())) == expect
+    assert n < 65 or gaps > 0
     g.close()
