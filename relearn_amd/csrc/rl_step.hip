@@ -146,6 +146,12 @@ __device__ __forceinline__ void push_out_pairs(const StepArgs& a, const uint2* p
     }
 }
 
+// One wave per block: a wave starts when its own registers are free and waits for no other, and a small
+// network's waves lie on compute units of their own.  Period of 100 steps with 64, 128, 256 and 512 threads per block:
+// 1,000 neurons 770, 784, 820 and 917 us; 300,001 neurons 2,355, 2,418, 2,409 and 2,480 us; 2M neurons
+// 11.34, 11.38, 11.49 and 11.66 ms.  Registers held to 8 waves per SIMD (64): 865, 2,515 us and 11.84 ms.
+constexpr int kStepBlock = 64;
+
 // One step of one neuron per lane.
 //
 // At 1M neurons the kernel moves its 106 bytes per neuron at 4.2 TB/s, 0.8 of what a device copy
@@ -160,11 +166,11 @@ __device__ __forceinline__ void push_out_pairs(const StepArgs& a, const uint2* p
 // for another, so a captured period's steps share launches: period of 100 steps without synaptic input
 // 676 -> 393 us for 1,000 neurons, 2,170 -> 1,622 us for 300,001, 10.63 -> 8.55 ms for 2M.
 template <uint32_t kSub, bool kSynaptic, bool kMany>
-__global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
+__global__ void __launch_bounds__(kStepBlock) k_step(StepArgs a) {
 #pragma clang fp contract(off)
     __shared__ double2 table[32];
     const uint32_t n = static_cast<uint32_t>(a.n);
-    const uint32_t lane_i = blockIdx.x * static_cast<uint32_t>(kBlock) + threadIdx.x;
+    const uint32_t lane_i = blockIdx.x * static_cast<uint32_t>(kStepBlock) + threadIdx.x;
     const bool in = lane_i < n;
     const uint32_t i = in ? lane_i : n - 1U;
     const rl_step_params& p = a.p;
@@ -309,9 +315,9 @@ constexpr uint32_t kStepsPerLaunch = 256;   // 60 ms for 16M neurons
 template <bool kSynaptic, bool kMany>
 void launch_step_of(const StepArgs& a, hipStream_t s) {
     if (a.p.h == 10) {
-        k_step<10, kSynaptic, kMany><<<grid_for(a.n), kBlock, 0, s>>>(a);
+        k_step<10, kSynaptic, kMany><<<grid_for(a.n, kStepBlock), kStepBlock, 0, s>>>(a);
     } else {
-        k_step<0, kSynaptic, kMany><<<grid_for(a.n), kBlock, 0, s>>>(a);
+        k_step<0, kSynaptic, kMany><<<grid_for(a.n, kStepBlock), kStepBlock, 0, s>>>(a);
     }
 }
 
