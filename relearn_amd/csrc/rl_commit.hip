@@ -370,7 +370,8 @@ __global__ void __launch_bounds__(kCountThreads) k_noalloc_take(uint32_t group_b
         const bool head = lane == 0 || s != before;   // lanes beyond m accept nothing, whatever run they join
         const uint64_t heads = __ballot(head);
         const uint64_t above = lane == 63 ? 0 : heads >> (lane + 1U);
-        const uint32_t length = above == 0 ? 64U - lane : static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(above)));
+        const uint32_t length =
+            above == 0 ? 64U - lane : static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(above)));
         const uint64_t run = length == 64U ? ~0ULL : ((1ULL << length) - 1ULL) << lane;
         const uint32_t taken = head ? static_cast<uint32_t>(__popcll(accepted & run)) : 0U;
         if (taken != 0) {

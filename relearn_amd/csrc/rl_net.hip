@@ -717,8 +717,8 @@ int enqueue_net_merge(rl_bh_ctx* c) {
     NetGraph& g = c->net;
     const uint64_t n = c->n;
     hipStream_t s = c->stream;
-    k_net_stage<<<stream_blocks(c->slots_cap), kBlock, 0, s>>>(n, g.off, g.cap, c->req_off + n, c->req_ok, c->req_target, c->req_source, g.npre,
-                                                 g.ncnt, c->c_sidx, c->counters);
+    k_net_stage<<<stream_blocks(c->slots_cap), kBlock, 0, s>>>(n, g.off, g.cap, c->req_off + n, c->req_ok, c->req_target,
+                                                               c->req_source, g.npre, g.ncnt, c->c_sidx, c->counters);
     RL_HIP(c, hipGetLastError());
     k_net_merge<<<grid_for(n), kBlock, 0, s>>>(n, g.off, g.npre, g.src, g.w, c->c_sidx, c->signal, g.src2, g.w2, g.ncnt,
                                                c->counters);
