@@ -32,13 +32,13 @@
 #include <algorithm>
 
 #include "rl_search_eval.h"
+#include "rl_slot_table.h"
 
 namespace rl {
 namespace {
 
 constexpr int kWave = 64;
 constexpr int kXcds = kCursorSlots;
-constexpr uint32_t kFxSlot = 0x7FFU;   // slot bits of an fx entry
 
 struct CoopArgs {
     SearchArgs s;
@@ -49,7 +49,7 @@ struct CoopArgs {
     uint32_t* t_my;               // per wave: cap slots, of which those that left the LDS ring are used
     uint32_t* t_fexp;
     double* t_mass;
-    uint32_t cap;                 // at most 2,048: slots fit the 11 bits of fx
+    uint32_t cap;                 // records per wave, more than kMostSlots
     uint32_t* overflow;
     unsigned long long* n_overflow;
     uint4* slow;                  // (slot, source, node, level) of descents for the per-lane kernel
@@ -69,14 +69,12 @@ struct CoopArgs {
 // tracked in every step and the reference's formulas inlined, a step took about 150 instructions and
 // the FP32-mixed kernel 96 VGPRs (5 waves per SIMD); now 105 and 80 (6 waves, 22 per CU by LDS).  1M
 // neurons: FP32-mixed 12.1 -> 8.8 ms, FP64 16.0 -> 11.5 ms.
-constexpr uint32_t kRing = 512;
-constexpr uint32_t kRingMask = kRing - 1U;
 template <bool kMixed>
 struct CoopShared {
     double ms[kRing];
     double2 exp_table[kMixed ? 1 : 32]; // 2^(i/32), first and second part (FP64 search only)
     uint32_t my[kRing];
-    uint16_t fx[kRing];                 // first expanded child's slot (if any) | expanded children << 11
+    uint16_t fx[kRing];                 // fx_pack(first expanded child's slot, expanded children)
 };
 
 __device__ __forceinline__ uint32_t lane() {
@@ -310,7 +308,6 @@ struct SlotTable {   // the global part, indexed by slot
     uint32_t* my;
     uint32_t* fx;
     double* ms;
-    uint32_t dump;   // one past the last slot
 };
 
 // Reads the entries [kb, min(kb + 8, tail)) of the queue and issues the loads of their children.
@@ -334,11 +331,12 @@ __device__ __forceinline__ StepIn fetch_step(const Lane& L, const CoopShared<kMi
 struct BfsState {
     uint32_t nslots;   // queue tail = slots allocated
     uint32_t out;      // slots below left the ring for the global table
+    uint32_t limit;    // slot_limit(out)
 };
 
 // Tests the children of one step's entries, sums the accepted probabilities per group, appends the
 // expanded children to the table and records the entries' masses.  Ends the traversal when the table would
-// overflow, or the ring with slots not yet processed.
+// overflow, which is tested in every step by way of b.limit, or the ring with slots not yet processed.
 template <bool kMixed, bool kMu0>
 __device__ __forceinline__ void bfs_step(const CoopArgs& a, const Lane& L, CoopShared<kMixed>& sh, const SlotTable& t,
                                          const StepIn& x, BfsState& b, Bfs& r) {
@@ -358,11 +356,10 @@ __device__ __forceinline__ void bfs_step(const CoopArgs& a, const Lane& L, CoopS
         const uint32_t gem = static_cast<uint32_t>(em >> (8U * q)) & 0xFFU;
         const uint32_t gi = x.k & kRingMask;
         sh.ms[gi] = gsum;
-        sh.fx[gi] = static_cast<uint16_t>(slot | (static_cast<uint32_t>(__popc(gem)) << 11U));
+        sh.fx[gi] = static_cast<uint16_t>(fx_pack(slot, static_cast<uint32_t>(__popc(gem))));
     }
-    if (tail > b.out + kRing) {
-        // 64 processed slots leave the ring (a step adds at most 64)
-        if (tail > t.dump || b.out + kWave > x.end) {
+    if (tail > b.limit) {
+        if (!slots_can_leave(tail, b.out, x.end)) {
             r.overflow = true;
             b.nslots = 0;   // ends the traversal
             return;
@@ -371,7 +368,8 @@ __device__ __forceinline__ void bfs_step(const CoopArgs& a, const Lane& L, CoopS
         at(t.my, sl) = sh.my[sl & kRingMask];
         at(t.fx, sl) = sh.fx[sl & kRingMask];
         at(t.ms, sl) = sh.ms[sl & kRingMask];
-        b.out += kWave;
+        b.out += kLeave;
+        b.limit = slot_limit(b.out);
     }
     if (__builtin_amdgcn_inverse_ballot_w64(em)) {
         sh.my[slot & kRingMask] = x.nd.m.y;
@@ -392,12 +390,11 @@ __device__ Bfs bfs(const CoopArgs& a, const Lane& L, uint32_t root_meta_y, CoopS
     t.my = a.t_my + base;
     t.fx = a.t_fexp + base;
     t.ms = a.t_mass + base;
-    t.dump = a.cap - 1;
     if (ln == 0) {
         sh.my[0] = root_meta_y;
     }
     __syncthreads();
-    BfsState b{ 1U, 0U };
+    BfsState b{ 1U, 0U, slot_limit(0U) };
     StepIn xa = fetch_step<kMixed, kMu0>(L, sh, 0U, 1U);
     // Wait for the first step's data here, so that the loop header carries no pending load.
     if (kMixed) {
@@ -425,9 +422,8 @@ __device__ Bfs bfs(const CoopArgs& a, const Lane& L, uint32_t root_meta_y, CoopS
         return r;
     }
     __syncthreads();
-    // Pull the masses of expanded children into their parents, last slots first, up to 64 at a time: the
-    // slots [lo, hi) above the last one of the 64 with a child below hi.  All their children lie at or beyond
-    // hi and have their final masses; slot hi - 1 always is one of them, since children follow parents.
+    // Pull the masses of expanded children into their parents, last slots first, up to 64 at a time: all
+    // children of the slots [lo, hi) lie at or beyond hi and have their final masses.
     *out = b.out;
     uint32_t hi = __builtin_amdgcn_readfirstlane(b.nslots);
     while (hi > 0) {
@@ -438,10 +434,9 @@ __device__ Bfs bfs(const CoopArgs& a, const Lane& L, uint32_t root_meta_y, CoopS
         if (sl < hi) {
             fx = in_lds || sl >= b.out ? sh.fx[sl & kRingMask] : at(t.fx, sl);
         }
-        const uint32_t f = fx & kFxSlot;
-        const uint32_t ne = fx >> 11U;
-        const uint64_t open = __builtin_amdgcn_ballot_w64(ne != 0 && f < hi);
-        const uint32_t lo = open == 0 ? first : first + kWave - static_cast<uint32_t>(__builtin_clzll(open));
+        const uint32_t f = fx_slot(fx);
+        const uint32_t ne = fx_count(fx);
+        const uint32_t lo = pull_from(first, __builtin_amdgcn_ballot_w64(ne != 0 && f < hi));
         if (sl >= lo && ne != 0) {
             double m8[8];
             if (in_lds) {
@@ -495,7 +490,7 @@ __device__ uint32_t navigate(const CoopArgs& a, const Lane& L, const CoopShared<
         if (__ballot(!done) == 0) {
             break;
         }
-        // slot < cap always holds: it only advances to a checked child slot
+        // slot < kMostSlots always holds: it only advances to a checked child slot
         uint32_t fx, my;
         if (__builtin_amdgcn_ballot_w64(slot < out) == 0) {
             fx = sh.fx[slot & kRingMask];
@@ -510,8 +505,8 @@ __device__ uint32_t navigate(const CoopArgs& a, const Lane& L, const CoopShared<
         }
         const uint32_t fc = my & kLinkMask;
         const uint32_t nc = my >> kLinkBits;
-        const uint32_t f = fx & kFxSlot;
-        const uint32_t nexp = fx >> 11U;
+        const uint32_t f = fx_slot(fx);
+        const uint32_t nexp = fx_count(fx);
         const bool act = !done && j < nc;
         // the children and the masses of the expanded ones, loaded together
         const NodeData nd = load_node<kMixed, kMu0>(L, fc + j, act);
@@ -555,7 +550,7 @@ __device__ uint32_t navigate(const CoopArgs& a, const Lane& L, const CoopShared<
             } else {
                 rr = rr - before;
                 const uint32_t next = f + static_cast<uint32_t>(__popc(gem & ((1U << jstar) - 1U)));
-                if (nexp == 0 || next >= a.cap - 1) {
+                if (nexp == 0 || next >= kMostSlots) {
                     done = true;
                     res = kNone;
                 } else {
