@@ -353,7 +353,7 @@ int init_networks(rl_bh_ctx* c, uint32_t G, const uint64_t* offsets, const doubl
             c->waves_per_cu = 24;   // the group walk's tables and LDS are sized for 24 waves per CU
         }
         c->coop_blocks = c->cus * c->waves_per_cu;
-        c->coop_cap = kMostSlots + 1;
+        c->coop_cap = kSlotRecords;
         if (!uses_walk(c) || walk_min_sources(c) > 0) {
             // the wave-per-source kernel (an FP32-mixed context with the group walk uses it for
             // updates with few active sources)

@@ -46,10 +46,10 @@ struct CoopArgs {
     const uint64_t* nwork;        // device count of work; XCD segment x is [nwork x / 8, nwork (x + 1) / 8)
     unsigned long long* cursor;   // kXcds counters
     uint32_t chunk;               // sources taken from a segment per cursor increment
-    uint32_t* t_my;               // per wave: cap slots, of which those that left the LDS ring are used
+    uint32_t* t_my;               // per wave: cap slots, of which those outside the LDS ring are used
     uint32_t* t_fexp;
     double* t_mass;
-    uint32_t cap;                 // records per wave, more than kMostSlots
+    uint32_t cap;                 // records per wave: kSlotRecords
     uint32_t* overflow;
     unsigned long long* n_overflow;
     uint4* slow;                  // (slot, source, node, level) of descents for the per-lane kernel
@@ -59,16 +59,21 @@ struct CoopArgs {
 
 // The slot table of the source a wave works on: per expanded node its packed child range (which also makes
 // the table the traversal's queue), the slot of its first expanded child with their number, and its
-// mass.  LDS holds the last kRing slots at slot % kRing, the wave's part of the global table the ones
-// before: a source expands about 110 nodes at 1,000 neurons, 340 at 52,000, 550 at 1M and 640 at 4M
-// (theta 0.3), so few slots or none leave the ring, and those are the top of the tree.
+// mass.  LDS holds a ring of kRing slots, the wave's part of the global table the others: a source expands
+// about 110 nodes at 1,000 neurons, 340 at 52,000, 550 at 1M and 640 at 4M (theta 0.3), so few slots or
+// none leave the ring, and those are the top of the tree.
+//
+// A level has up to about 4/3 pi / theta^3 expanded nodes: 155 at theta 0.3, 393 at 0.22, 523 at 0.2, so at
+// small theta more slots wait than the ring holds.  They wait in the global table.  While such sources were
+// handed to the per-lane search, the 1M-neuron update took 87.8 ms at theta 0.22 (a quarter of the sources),
+// now 19.2, and 106.2 ms in FP64, now 24.8.  Sources that need more than the table are handed over still.
 //
 // What bounds the search is the number of instructions of any kind that a wave issues one after another
 // (1.7 per cycle and SIMD at 5 waves, vector and scalar units 70% busy each), not one unit and not
 // memory.  With the whole table in global memory behind LDS staging rings, the level boundaries
 // tracked in every step and the reference's formulas inlined, a step took about 150 instructions and
 // the FP32-mixed kernel 96 VGPRs (5 waves per SIMD); now 105 and 80 (6 waves, 22 per CU by LDS).  1M
-// neurons: FP32-mixed 12.1 -> 8.8 ms, FP64 16.0 -> 11.5 ms.
+// neurons: FP32-mixed 12.1 -> 8.7 ms, FP64 16.0 -> 11.4 ms.
 template <bool kMixed>
 struct CoopShared {
     double ms[kRing];
@@ -329,14 +334,15 @@ __device__ __forceinline__ StepIn fetch_step(const Lane& L, const CoopShared<kMi
 }
 
 struct BfsState {
-    uint32_t nslots;   // queue tail = slots allocated
+    uint32_t nslots;   // queue tail = slots allocated; 0 after a step that went beyond the limit, and then
+    uint32_t tail;     // the slots allocated
     uint32_t out;      // slots below left the ring for the global table
     uint32_t limit;    // slot_limit(out)
 };
 
 // Tests the children of one step's entries, sums the accepted probabilities per group, appends the
-// expanded children to the table and records the entries' masses.  Ends the traversal when the table would
-// overflow, which is tested in every step by way of b.limit, or the ring with slots not yet processed.
+// expanded children to the ring and records the entries' masses.  In a step that goes beyond b.limit, those for
+// which the ring has no room wait in the global table, and bfs() has to make room or give up.
 template <bool kMixed, bool kMu0>
 __device__ __forceinline__ void bfs_step(const CoopArgs& a, const Lane& L, CoopShared<kMixed>& sh, const SlotTable& t,
                                          const StepIn& x, BfsState& b, Bfs& r) {
@@ -359,17 +365,16 @@ __device__ __forceinline__ void bfs_step(const CoopArgs& a, const Lane& L, CoopS
         sh.fx[gi] = static_cast<uint16_t>(fx_pack(slot, static_cast<uint32_t>(__popc(gem))));
     }
     if (tail > b.limit) {
-        if (!slots_can_leave(tail, b.out, x.end)) {
-            r.overflow = true;
-            b.nslots = 0;   // ends the traversal
-            return;
+        if (__builtin_amdgcn_inverse_ballot_w64(em)) {
+            if (slot < b.out + kRing) {
+                sh.my[slot & kRingMask] = x.nd.m.y;
+            } else {
+                at(t.my, slot) = x.nd.m.y;
+            }
         }
-        const uint32_t sl = b.out + ln;
-        at(t.my, sl) = sh.my[sl & kRingMask];
-        at(t.fx, sl) = sh.fx[sl & kRingMask];
-        at(t.ms, sl) = sh.ms[sl & kRingMask];
-        b.out += kLeave;
-        b.limit = slot_limit(b.out);
+        b.tail = tail;
+        b.nslots = 0;
+        return;
     }
     if (__builtin_amdgcn_inverse_ballot_w64(em)) {
         sh.my[slot & kRingMask] = x.nd.m.y;
@@ -394,7 +399,7 @@ __device__ Bfs bfs(const CoopArgs& a, const Lane& L, uint32_t root_meta_y, CoopS
         sh.my[0] = root_meta_y;
     }
     __syncthreads();
-    BfsState b{ 1U, 0U, slot_limit(0U) };
+    BfsState b{ 1U, 1U, 0U, slot_limit(0U) };
     StepIn xa = fetch_step<kMixed, kMu0>(L, sh, 0U, 1U);
     // Wait for the first step's data here, so that the loop header carries no pending load.
     if (kMixed) {
@@ -404,17 +409,44 @@ __device__ Bfs bfs(const CoopArgs& a, const Lane& L, uint32_t root_meta_y, CoopS
         __asm__ volatile("" ::"v"(xa.nd.m.x), "v"(xa.nd.m.y), "v"(xa.nd.r64.x), "v"(xa.nd.r64.y), "v"(xa.nd.r64.z),
                          "v"(xa.nd.r64.w));
     }
+    // After a step whose successor starts at slot `next`, when that is no slot: the traversal ends, or the step
+    // went beyond the limit.  Both share the exit test, and the room is made out of the step, whose registers it
+    // would take: 18 more spilled in the FP32-mixed kernel.  1M neurons at theta 0.3: 8.67 ms FP32-mixed and
+    // 11.40 FP64, against 8.80 and 11.43 with the room made in the step and no slots outside the ring.
+    auto ends = [&](uint32_t next) -> bool {
+        if (b.nslots != 0) {
+            return true;
+        }
+        if (b.tail > kMostSlots) {
+            r.overflow = true;
+            return true;
+        }
+        if (slots_leave(b.out, next)) {
+            const uint32_t sl = b.out + ln;
+            at(t.my, sl) = sh.my[sl & kRingMask];
+            at(t.fx, sl) = sh.fx[sl & kRingMask];
+            at(t.ms, sl) = sh.ms[sl & kRingMask];
+            if (sl + kRing < b.tail) {   // a slot that waits outside takes the place
+                __threadfence_block();
+                sh.my[sl & kRingMask] = at(t.my, sl + kRing);
+            }
+            b.out += kLeave;
+            b.limit = slot_limit(b.out);
+        }
+        b.nslots = b.tail;
+        return next >= b.nslots;
+    };
     while (true) {
-        StepIn xb = fetch_step<kMixed, kMu0>(L, sh, xa.end, b.nslots);
+        const StepIn xb = fetch_step<kMixed, kMu0>(L, sh, xa.end, b.nslots);
         __builtin_amdgcn_sched_barrier(0);   // keep the prefetch ahead of this step's work
         bfs_step<kMixed, kMu0>(a, L, sh, t, xa, b, r);
-        if (xb.kb >= b.nslots) {
+        if (xb.kb >= b.nslots && ends(xb.kb)) {
             break;
         }
         xa = fetch_step<kMixed, kMu0>(L, sh, xb.end, b.nslots);
         __builtin_amdgcn_sched_barrier(0);
         bfs_step<kMixed, kMu0>(a, L, sh, t, xb, b, r);
-        if (xa.kb >= b.nslots) {
+        if (xa.kb >= b.nslots && ends(xa.kb)) {
             break;
         }
     }

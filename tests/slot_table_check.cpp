@@ -56,9 +56,8 @@ int main(int argc, char** argv) {
     std::mt19937 gen(static_cast<uint32_t>(std::atoi(argv[3])));
     const std::vector<uint32_t> kids = tree(slots, waiting, argc > 4, gen);
 
-    constexpr uint32_t kRecords = kMostSlots + 1;
-    std::vector<double> ms(kRing, -1.0), t_ms(kRecords, -1.0);
-    std::vector<uint32_t> my(kRing, ~0U), t_my(kRecords, ~0U), t_fx(kRecords, ~0U);
+    std::vector<double> ms(kRing, -1.0), t_ms(kSlotRecords, -1.0);
+    std::vector<uint32_t> my(kRing, ~0U), t_my(kSlotRecords, ~0U), t_fx(kSlotRecords, ~0U);
     std::vector<uint16_t> fx(kRing, 0xFFFF);
     // an entry of the queue stands for its own slot number, its mass is 1
     uint32_t tail = 1, out = 0, limit = slot_limit(0), most_waiting = 0;
@@ -82,27 +81,32 @@ int main(int argc, char** argv) {
             ms[k & kRingMask] = 1.0;
             to += kids[k];
         }
-        if (to > limit) {
-            if (!slots_can_leave(to, out, end)) {
-                std::printf("overflow %u %u\n", to, most_waiting);
-                return 0;
-            }
-            for (uint32_t s = out; s < out + kLeave; s++) {
-                t_my[s] = my[s & kRingMask];
-                t_fx[s] = fx[s & kRingMask];
-                t_ms[s] = ms[s & kRingMask];
-            }
-            out += kLeave;
-            limit = slot_limit(out);
-        }
         for (uint32_t s = before; s < to; s++) {
-            if (s >= kRecords || s - out >= kRing) {
+            if (s >= kSlotRecords || (to <= limit && s >= out + kRing)) {
                 return fail("slot out of range", s);
             }
-            my[s & kRingMask] = s;
+            (to <= limit || s < out + kRing ? my[s & kRingMask] : t_my[s]) = s;
         }
         tail = to;
         most_waiting = std::max(most_waiting, tail - end);
+        if (tail > limit) {
+            if (tail > kMostSlots) {
+                std::printf("overflow %u %u\n", tail, most_waiting);
+                return 0;
+            }
+            if (slots_leave(out, end)) {
+                for (uint32_t s = out; s < out + kLeave; s++) {
+                    t_my[s] = my[s & kRingMask];
+                    t_fx[s] = fx[s & kRingMask];
+                    t_ms[s] = ms[s & kRingMask];
+                    if (s + kRing < tail) {
+                        my[s & kRingMask] = t_my[s + kRing];
+                    }
+                }
+                out += kLeave;
+                limit = slot_limit(out);
+            }
+        }
         if (end >= tail) {
             break;
         }

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from relearn_amd import RL_PREC_FP32_MIXED, RL_PREC_FP64
-from relearn_amd.workloads import Network
+from relearn_amd.workloads import Network, uniform_cube
 from tests.test_gpu_parity import _check_search, _search_pair
 
 pytestmark = pytest.mark.gpu
@@ -73,4 +73,17 @@ def test_search_parity_at_the_tables_end(oracle, precision):
     assert ((slots >= 1900) & (slots <= MOST)).sum() > 100 and (slots > MOST).sum() > 100
     for k in (MOST - 1, MOST, MOST + 1, MOST + 2):
         assert (slots == k).any()
+    assert lane_sources == (slots > MOST).sum()
+
+
+@pytest.mark.parametrize("theta", [0.2, 0.15])
+@pytest.mark.parametrize("precision", [RL_PREC_FP64, RL_PREC_FP32_MIXED])
+def test_search_parity_with_levels_wider_than_the_ring(oracle, precision, theta):
+    print("[gpu-case] slot table, uniform 52,000, theta", theta, "precision", precision, flush=True)
+    net = uniform_cube(52_000, 10_000.0 * (0.052 ** (1 / 3)), 4)
+    net.vac_axon[np.arange(net.n) % 32 != 0] = 0
+    counts, lane_sources = _run(oracle, net, theta, precision)
+    slots, widest = counts[:, 0], counts[:, 1]
+    assert (widest[slots <= MOST] > 520).sum() > 50   # more than the ring's 512 slots wait at once
+    assert (slots > MOST).any() == (theta == 0.15)
     assert lane_sources == (slots > MOST).sum()

@@ -37,3 +37,14 @@ def test_slot_table_ends(check, slots, waiting):
     for seed in range(8):
         for end_full in (False, True):
             assert check(slots, waiting, seed, end_full)[0] == ("done" if slots <= MOST else "overflow")
+
+
+# more waiting slots than the ring holds: they wait in the table
+@pytest.mark.parametrize("slots", [600, 1024, 2046, 2047, 2048, 2049])
+@pytest.mark.parametrize("waiting", [447, 448, 449, 504, 512, 520, 600, 1000, 2000])
+def test_slots_that_wait_outside_the_ring(check, slots, waiting):
+    for seed in range(8):
+        kind, _, most = check(slots, waiting, seed)
+        assert kind == ("done" if slots <= MOST else "overflow")
+        if slots >= MOST - 1:
+            assert int(most) >= min(waiting, 1200)
