@@ -332,8 +332,6 @@ hipError_t scan_counts_on(hipStream_t s, const uint32_t* in, uint64_t n, uint64_
                           uint64_t* total = nullptr);
 int fill_u32(rl_bh_ctx* c, uint32_t* p, uint32_t value, uint64_t n);
 int set_steps(rl_bh_ctx* c, uint32_t neuron_step, uint32_t update);
-// The device's address of a page-locked host range, or null (pageable, device or managed memory).
-void* mapped_host(const void* p, size_t bytes);
 // Arrays of one API call, copied on the context's stream.
 struct CopyItem {
     void* dst;

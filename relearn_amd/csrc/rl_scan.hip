@@ -5,6 +5,7 @@
 // depend on timing.
 #include <algorithm>
 
+#include "rl_caller_memory.h"
 #include "rl_internal.h"
 
 namespace rl {
@@ -322,40 +323,6 @@ int fill_u32(rl_bh_ctx* c, uint32_t* p, uint32_t value, uint64_t n) {
     return RL_OK;
 }
 
-void* mapped_host(const void* p, size_t bytes) {
-    if (p == nullptr || bytes == 0) {
-        return nullptr;
-    }
-    const char* const end = static_cast<const char*>(p) + bytes - 1;
-    hipPointerAttribute_t first{}, last{};
-    if (hipPointerGetAttributes(&first, p) != hipSuccess || hipPointerGetAttributes(&last, end) != hipSuccess) {
-        (void)hipGetLastError();   // memory that HIP does not know
-        return nullptr;
-    }
-    if (first.type != hipMemoryTypeHost || last.type != hipMemoryTypeHost || first.devicePointer == nullptr ||
-        static_cast<char*>(last.devicePointer) - static_cast<char*>(first.devicePointer) !=
-            static_cast<ptrdiff_t>(bytes - 1)) {
-        return nullptr;
-    }
-    return first.devicePointer;
-}
-
-namespace {
-
-// Device memory of the context's own GPU.
-bool own_device(const rl_bh_ctx* c, const void* p, size_t bytes) {
-    hipPointerAttribute_t first{}, last{};
-    if (hipPointerGetAttributes(&first, p) != hipSuccess ||
-        hipPointerGetAttributes(&last, static_cast<const char*>(p) + bytes - 1) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return first.type == hipMemoryTypeDevice && last.type == hipMemoryTypeDevice && first.device == c->cfg.device &&
-           last.device == c->cfg.device;
-}
-
-}  // namespace
-
 // One launch for the arrays that the device can address (page-locked host arrays, memory of the own GPU);
 // the rest by copies.  Each copy of its own costs 9 to 10 us whatever its size: with one launch per
 // call, and the counts written to page-locked memory by the kernels that form them, a 1,000-neuron update
@@ -376,7 +343,7 @@ int copy_arrays(rl_bh_ctx* c, const CopyItem* items, int count, hipMemcpyKind ki
             src = mapped_host(it.src, it.bytes);
         } else if (kind == hipMemcpyDeviceToHost) {
             dst = mapped_host(it.dst, it.bytes);
-        } else if (!own_device(c, it.src, it.bytes)) {
+        } else if (!own_device(c->cfg.device, it.src, it.bytes)) {
             src = nullptr;
         }
         if (src == nullptr || dst == nullptr || listed == kMaxCopies) {

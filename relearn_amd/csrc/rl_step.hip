@@ -12,6 +12,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "rl_caller_memory.h"
 #include "rl_device.h"
 #include "rl_internal.h"
 
