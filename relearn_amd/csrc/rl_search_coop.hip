@@ -368,7 +368,7 @@ __device__ __forceinline__ void bfs_step(const CoopArgs& a, const Lane& L, CoopS
             if (slot < b.out + kRing) {
                 sh.my[slot & kRingMask] = x.nd.m.y;
             } else {
-                at(t.my, slot) = x.nd.m.y;
+                at(t.my, waiting_record(slot)) = x.nd.m.y;
             }
         }
         b.tail = tail;

@@ -20,9 +20,10 @@ constexpr uint32_t kRing = 512;
 constexpr uint32_t kRingMask = kRing - 1U;
 constexpr uint32_t kLeave = 64;            // slots that leave the ring together; a step adds at most as many
 // Slots of a source: every slot number up to and including the number of slots, which a node without expanded
-// children records, fits the 11 bits of an fx entry.  The table has room for one more step, which finds out.
+// children records, fits the 11 bits of an fx entry.  The table's last record takes the slots beyond of the step
+// that needs more.
 constexpr uint32_t kMostSlots = 2047;
-constexpr uint32_t kSlotRecords = kMostSlots + 1 + kLeave;
+constexpr uint32_t kSlotRecords = kMostSlots + 1;
 
 // What a slot records of its children: the slot of the first expanded one and how many there are.
 RL_BOTH uint32_t fx_pack(uint32_t slot, uint32_t count) { return slot | count << 11U; }
@@ -31,6 +32,9 @@ RL_BOTH uint32_t fx_count(uint32_t fx) { return fx >> 11U; }
 
 // The number of slots up to which a step appends to the ring as it is: the end of the ring, and of the table.
 RL_BOTH uint32_t slot_limit(uint32_t out) { return out + kRing < kMostSlots ? out + kRing : kMostSlots; }
+
+// The record in which a slot waits outside the ring.
+RL_BOTH uint32_t waiting_record(uint32_t slot) { return slot < kMostSlots ? slot : kMostSlots; }
 
 // Whether the first kLeave slots leave the ring after a step that processed the slots before `end` and went
 // beyond slot_limit(out).  While slots wait outside, that is asked after every step, and a step processes 8:

@@ -82,10 +82,10 @@ int main(int argc, char** argv) {
             to += kids[k];
         }
         for (uint32_t s = before; s < to; s++) {
-            if (s >= kSlotRecords || (to <= limit && s >= out + kRing)) {
+            if (waiting_record(s) >= kSlotRecords || (to <= limit && s >= out + kRing)) {
                 return fail("slot out of range", s);
             }
-            (to <= limit || s < out + kRing ? my[s & kRingMask] : t_my[s]) = s;
+            (to <= limit || s < out + kRing ? my[s & kRingMask] : t_my[waiting_record(s)]) = s;
         }
         tail = to;
         most_waiting = std::max(most_waiting, tail - end);
