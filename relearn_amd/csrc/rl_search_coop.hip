@@ -68,12 +68,12 @@ struct CoopArgs {
 // handed to the per-lane search, the 1M-neuron update took 87.8 ms at theta 0.22 (a quarter of the sources),
 // now 19.2, and 106.2 ms in FP64, now 24.8.  Sources that need more than the table are handed over still.
 //
-// What bounds the search is the number of instructions of any kind that a wave issues one after another
-// (1.7 per cycle and SIMD at 5 waves, vector and scalar units 70% busy each), not one unit and not
-// memory.  With the whole table in global memory behind LDS staging rings, the level boundaries
+// What bounds the search are its vector instructions (units 0.99 busy at 1M neurons, both precisions) and the data
+// path of its loads (0.97), so every instruction of a step counts; the scalar unit is 0.58 busy, L2 hits
+// 0.97.  With the whole table in global memory behind LDS staging rings, the level boundaries
 // tracked in every step and the reference's formulas inlined, a step took about 150 instructions and
 // the FP32-mixed kernel 96 VGPRs (5 waves per SIMD); now 105 and 80 (6 waves, 22 per CU by LDS).  1M
-// neurons: FP32-mixed 12.1 -> 8.7 ms, FP64 16.0 -> 11.4 ms.
+// neurons: FP32-mixed 12.1 -> 8.7 ms, FP64 16.0 -> 11.3 ms.
 template <bool kMixed>
 struct CoopShared {
     double ms[kRing];
@@ -207,7 +207,7 @@ constexpr double kTiny = 1.0e-250;
 // reference's; the Gaussian takes d^2 itself, which is rounded less than the square of the reference's
 // scaled hypot.  That hypot (three divisions and a square root, about 75 of the 210 vector
 // instructions of an FP64 step) and the library's exp made the FP64 search of 1M neurons 24.4 ms; with
-// squares and exp_gauss it takes 16.0 ms (and 11.5 with the ring table below).
+// squares and exp_gauss it takes 16.0 ms (and 11.3 with the ring table above).
 template <bool kMixed, bool kMu0>
 __device__ __forceinline__ Verdict eval_node(const SearchArgs& a, const Lane& L, const NodeData& d, uint32_t node,
                                              uint64_t act, const double2* table, double* p_out) {

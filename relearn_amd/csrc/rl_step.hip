@@ -1,7 +1,7 @@
 // Fused per-step neuron update: background input, Izhikevich membrane update, calcium integrator and
 // the growth-curve deltas of the three synaptic element types, one lane per neuron, in FP64 (the
-// counter-based background draw, normal_input below, is FP32) and in the CPU path's operation order
-// (files compiled with -ffp-contract=off):
+// counter-based background draw, normal_input below, is FP32) and in the CPU path's operation order, but for
+// the growth curves' exponential, which is exp_gauss (files compiled with -ffp-contract=off):
 //   IzhikevichModelCPU::update_activity   (source/neurons/models/izhikevich/IzhikevichModelCPU.cpp:75-125)
 //   CalciumCalculatorCPU::update_current_calcium (source/neurons/calcium/CalciumCalculatorCPU.cpp:40-103)
 //   update_number_elements_openmp + gaussian_growth_curve
@@ -112,6 +112,9 @@ __device__ __forceinline__ const T& at(const T* base, uint32_t i) {
 // 2,410 with 16; 1,000 neurons 955, 929, 874, 828 and 834 us; 2M neurons 11.78, 11.69, 11.70, 11.74 and 11.96 ms.
 // With the loads free of branches, and skipped whole by waves in which no neuron fired, 1,000 neurons went
 // from 843 to 829 us and 2M from 11.42 to 11.33 ms.
+// 12 holds the whole list of a neuron with up to 12 partners, as the simulated networks of 3 to 10 synapses
+// per neuron have them; each further 8 pairs are a round trip more.  With 5, 12, 24 and 60 pairs per neuron the
+// period of 1,000 neurons takes 727, 815, 1,046 and 1,795 us, that of 300,001 2.34, 2.58, 3.03 and 4.69 ms.
 constexpr uint32_t kPushAhead = 12;
 constexpr uint32_t kPushBatch = 8;
 
